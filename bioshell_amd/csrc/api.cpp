@@ -114,6 +114,7 @@ bs_status bs_context_create(int device, size_t hbm_budget_bytes, bs_context** ou
         auto ctx = std::make_unique<bs_context>();
         ctx->device = device;
         ctx->n_cu = prop.multiProcessorCount;
+        BS_HIP(hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device));
         ctx->gsc.max_wg = 2 * ctx->n_cu;
         ctx->budget.set_cap(hbm_budget_bytes);
         BS_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));

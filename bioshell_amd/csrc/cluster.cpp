@@ -2,6 +2,8 @@
 // clustering tools consume: row minima / maxima and the agglomerative
 // clustering loop (kernels_cluster.hip).
 #include <algorithm>
+#include <cstring>
+#include <vector>
 
 #include "engine.hpp"
 
@@ -25,10 +27,59 @@ const float* upload_upper(bs_context* ctx, const float* upper, size_t n)
     return d;
 }
 
+// The one-launch loop.  False when the device would not take the launch (its
+// work-groups have to be resident together): the caller runs the stepwise loop.
+bool cluster_one_launch(bs_context* ctx, const AgglomPlan& plan, const float* d_upper, size_t n, int rule,
+                        uint32_t* merge_i, uint32_t* merge_j, float* merge_d)
+{
+    hipStream_t s = ctx->stream;
+    const int N = (int)n;
+    DevBuf D, aux;
+    D.bind(&ctx->budget);
+    aux.bind(&ctx->budget);
+    const size_t ld = (n + 63) / 64 * 64;
+    AgglomArgs a{};
+    a.D = static_cast<float*>(D.ensure(n * ld * 4, "clustering matrix"));
+    a.ld = (int64_t)ld;
+    a.n = N;
+    a.rule = rule;
+    // slots, status (with padding), merges, exchanged rows
+    const size_t o_status = (size_t)plan.groups * 3 * 8, o_merge = o_status + 16,
+                 o_new = (o_merge + n * 12 + 255) / 256 * 256;
+    char* p = static_cast<char*>(aux.ensure(o_new + ld * 12, "clustering state"));
+    a.slots = reinterpret_cast<uint64_t*>(p);
+    a.status = reinterpret_cast<unsigned*>(p + o_status);
+    a.mi = reinterpret_cast<unsigned*>(p + o_merge);
+    a.mj = a.mi + n;
+    a.md = reinterpret_cast<float*>(a.mj + n);
+    a.newrow = reinterpret_cast<float*>(p + o_new);
+    a.max_wait = (uint64_t)ctx->clock_khz * 5000;  // 5 s
+    launch_agglom_init(d_upper, N, (int)ld, a.D, reinterpret_cast<unsigned*>(p), (int)(o_merge / 4), s);
+    BS_HIP(hipGetLastError());
+    const hipError_t e = launch_agglom(plan, a, s);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        BS_HIP(hipStreamSynchronize(s));  // the buffers go
+        return false;
+    }
+    std::vector<uint32_t> h(4 + 3 * n);
+    BS_HIP(hipMemcpyAsync(h.data(), p + o_status, h.size() * 4, hipMemcpyDeviceToHost, s));
+    BS_HIP(hipStreamSynchronize(s));
+    if (h[0] != 0) fail(BS_ERR_INTERNAL, "clustering: a work-group waited too long for the others");
+    std::memcpy(merge_i, h.data() + 4, (n - 1) * 4);
+    std::memcpy(merge_j, h.data() + 4 + n, (n - 1) * 4);
+    std::memcpy(merge_d, h.data() + 4 + 2 * n, (n - 1) * 4);
+    return true;
+}
+
 void cluster_device(bs_context* ctx, const float* d_upper, size_t n, int rule, uint32_t* merge_i,
                     uint32_t* merge_j, float* merge_d)
 {
     if (n < 2) return;
+    AgglomPlan plan;
+    if (agglom_plan((int)n, ctx->n_cu, &plan) &&
+        cluster_one_launch(ctx, plan, d_upper, n, rule, merge_i, merge_j, merge_d))
+        return;
     hipStream_t s = ctx->stream;
     const int N = (int)n;
     const int n_part = std::max(1, std::min(4 * ctx->n_cu, (N + 3) / 4));

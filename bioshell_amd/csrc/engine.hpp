@@ -253,6 +253,7 @@ struct bs_context {
     std::vector<bs::TuneCell> tune[4];  // autotuner: Gram tile side per (L, n) cell, per method
     bs::BatchWorkspace batch;          // batched pipeline (bs_crmsd_batch*)
     int n_cu = 0;
+    int clock_khz = 0;                 // rate of the device's wall clock
     std::mutex mu;
 };
 

@@ -270,6 +270,32 @@ void launch_cluster_init(const float* up, int n, int ld, float* D, unsigned* siz
 void launch_cluster_step(float* D, int n, int ld, void* state, void* part, int n_part, unsigned* sizes,
                          int rule, unsigned* mi, unsigned* mj, float* md, hipStream_t s);
 
+// The same loop in one launch (kernels_agglom.hip), for the element counts
+// agglom_plan takes (about 15,000 on 256 CUs; the stepwise launches above run
+// the larger ones).  slots (3 x groups), newrow (3 x ld) and status are the
+// exchange buffers; slots and status are zero at the launch.
+struct AgglomArgs {
+    float* D;               // n rows of ld floats, ld a multiple of 64
+    int64_t ld;
+    int n, rule;
+    unsigned *mi, *mj;      // n - 1 each
+    float* md;
+    uint64_t* slots;
+    float* newrow;
+    unsigned* status;       // set when a wait ran into max_wait
+    uint64_t max_wait;      // ticks of the wall clock
+    int rows, n_blocks, block_shift;  // filled by launch_agglom from the plan
+};
+struct AgglomPlan {
+    int groups = 0, rows = 0;       // work-groups, rows each
+    int n_blocks = 0, block_shift = 0;  // cached minima per row, columns per minimum (log2)
+    size_t lds = 0;
+};
+bool agglom_plan(int n, int n_cu, AgglomPlan* out);
+// The dense matrix (+inf on the diagonal and past column n) and n_zero cleared words at zero.
+void launch_agglom_init(const float* up, int n, int ld, float* D, unsigned* zero, int n_zero, hipStream_t s);
+hipError_t launch_agglom(const AgglomPlan& p, AgglomArgs a, hipStream_t s);
+
 // Single-pair superposition (rotation + translation) in FP64.
 void launch_superpose(const double* a, const double* b, int L, double* out13, hipStream_t s);
 // Every conformation of xyz (n x L x 3) onto ref (L x 3): rot n x 9, trans

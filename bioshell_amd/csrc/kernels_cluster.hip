@@ -12,6 +12,7 @@
 // clustering_matrix.rs step for step on a dense f32 matrix in HBM (see the
 // comments at each phase); the merge sequence it records is what the host
 // rebuilds the tree from.
+#include "cluster_rule.hpp"
 #include "kernels.hpp"
 #include "wave.hpp"
 
@@ -216,32 +217,6 @@ __global__ void dense_from_upper_kernel(const float* __restrict__ up, int n, int
     }
     for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256)
         sizes[k] = 1u;
-}
-
-// The merging rules of strategies/mod.rs in f32, evaluated left to right with
-// no contraction into fused multiply-adds (every operation rounds, as in the
-// reference); the division is the correctly rounded f32 division.
-__device__ inline float merge_rule(int rule, unsigned si, unsigned sj, unsigned sk, float dij,
-                                   float dik, float djk)
-{
-#pragma clang fp contract(off)
-    switch (rule) {
-    case 0: return fminf(dik, djk);
-    case 1: return fmaxf(dik, djk);
-    case 2: {
-        const float d = 1.0f / (float)(si + sj);
-        return d * (float)si * dik + d * (float)sj * djk;
-    }
-    case 3: return 0.5f * dik + 0.5f * djk - 0.25f * dij;
-    case 4: {
-        const float d = 1.0f / (float)(si + sj);
-        return d * (float)si * dik + d * (float)sj * djk - (float)si * (float)sj * d * d * dij;
-    }
-    default: {
-        const float d = 1.0f / (float)(si + sj + sk);
-        return d * (float)(si + sk) * dik + d * (float)(sj + sk) * djk - (float)sk * d * dij;
-    }
-    }
 }
 
 // The decision of one merge, written by the last work-group of a launch and

@@ -262,3 +262,36 @@ def test_clustering_2000_timing(gpu_ctx):
     print(f"device clustering of {n}: {dt * 1e3:.1f} ms")
     assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
     assert np.array_equal(got[0], want[0].astype(np.uint32))
+
+
+@pytest.mark.parametrize("linkage", C.LINKAGES)
+@pytest.mark.parametrize("n", [2, 4, 47, 48, 49, 72, 127, 129, 257])
+def test_merges_with_infinities_zeros_and_nan(gpu_ctx, linkage, n):
+    """One work-group and several, block and row edges, on values that are
+    never taken (+inf, f32::MAX, NaN), on zeros of both signs, negative values
+    and heavy ties: the merges of the oracle."""
+    rng = np.random.default_rng(n)
+    k = n * (n - 1) // 2
+    up = rng.integers(-2, 3, k).astype(np.float32)
+    for v in (np.inf, np.nan, np.float32(-0.0), np.finfo(np.float32).max):
+        up[rng.random(k) < 0.06] = v
+    for x in (up, np.full(k, np.inf, np.float32)):
+        got = device_merges(gpu_ctx, x, n, linkage)
+        want = O.hclust(x, n, linkage)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        # heights as values: the maximum of -0 and +0 may be either
+        assert np.array_equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("n", [6200, 12100, 15800])
+def test_large_single_link_heights(gpu_ctx, n):
+    """Points on a line, single linkage: the heights are the sorted gaps.  The
+    sizes take every work-group, the wider blocks and the stepwise launches."""
+    rng = np.random.default_rng(n)
+    x = np.cumsum(rng.integers(1, 1000, n)).astype(np.float32)  # exact in f32, below 2^24
+    assert x[-1] < 2 ** 24
+    p = rng.permutation(n)
+    y = x[p]
+    up = np.concatenate([np.abs(y[i] - y[i + 1:]) for i in range(n - 1)])
+    _, _, md = device_merges(gpu_ctx, up, n, "single")
+    assert np.array_equal(md, np.sort(np.diff(x)))
