@@ -619,7 +619,7 @@ def main() -> None:
         step(B.Method.BF16X3_GRAM, d_out)
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
-    # per-step device times from the library's HIP events (on its stream)
+    # per-step device times, as the library's kernels stamp them
     hist = ctx.history(args.steps)
     main_ms = [h["main_ms"] for h in hist]
     prep_ms = [h["prep_ms"] for h in hist]

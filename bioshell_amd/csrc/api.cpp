@@ -59,10 +59,8 @@ void context_release(bs_context* ctx)
         (void)hipStreamSynchronize(ctx->stream);
         ctx->prep.reset();
         ctx->qws.reset();
-        for (auto& r : ctx->ring) r.destroy();
         ctx->ring.clear();
-        if (ctx->h_counts) (void)hipHostFree(ctx->h_counts);
-        ctx->h_counts = nullptr;
+        ctx->ws_clock.reset();
         ctx->gsc.reset();
         for (auto& b : ctx->stream_blk) b.reset();
         for (int k = 0; k < 2; ++k) {
@@ -126,6 +124,7 @@ bs_status bs_context_create(int device, size_t hbm_budget_bytes, bs_context** ou
         ctx->ws_out.bind(&ctx->budget);
         ctx->ws_misc.bind(&ctx->budget);
         ctx->ws_stats.bind(&ctx->budget);
+        ctx->ws_clock.bind(&ctx->budget);
         ctx->batch.bind(&ctx->budget);
         *out = ctx.release();
     });

@@ -270,17 +270,19 @@ void enqueue_plain(bs_context* ctx, const Plan& P, const std::vector<const doubl
         o_pre[g] = put(blob, pre[g].data(), pre[g].size() * 4);
     }
     char* meta = upload_meta(ctx->batch, blob, s);
-    rec->mark({kBTotal0, kBPrep0, kBPrep1, kBMain0}, s);
     uint64_t launches = 0;
+    int g_last = 2;
+    while (g_last > 0 && grp[g_last].empty()) --g_last;
     for (int g = 0; g < 3; ++g) {
         if (grp[g].empty()) continue;
         launch_plain_batch(reinterpret_cast<const PlainEns*>(meta + o_ens[g]),
                            reinterpret_cast<const int*>(meta + o_pre[g]), (int)grp[g].size(),
-                           pre[g].back(), 1 << g, fp64, s);
+                           pre[g].back(), 1 << g, fp64, s, launches == 0 ? rec->clk + kClkStart : nullptr,
+                           g == g_last ? rec->clk + kClkEnd : nullptr, rec->done);
         ++launches;
     }
     BS_HIP(hipGetLastError());
-    rec->mark({kBMain1, kBFallback0, kBFallback1, kBTotal1}, s);
+    rec->kind = RunRecord::kOneStage;
     rec->base.main_launches = launches;
 }
 
@@ -296,10 +298,7 @@ void enqueue(bs_context* ctx, const Plan& P, const std::vector<const double*>& d
     rec->base.pairs = P.pairs;
     rec->base.main_launches = 1;
     rec->base.tile_m = rec->base.tile_n = 0;
-    if (E == 0) {
-        rec->mark({kBTotal0, kBTotal1, kBPrep0, kBPrep1, kBMain0, kBMain1, kBFallback0, kBFallback1}, s);
-        return;
-    }
+    if (E == 0) return;
     if (!P.gram) {
         enqueue_plain(ctx, P, d_xyz, d_out, rec);
         return;
@@ -315,7 +314,7 @@ void enqueue(bs_context* ctx, const Plan& P, const std::vector<const double*>& d
     double* con = static_cast<double*>(W.consts.ensure((size_t)P.con_doubles * 8, "batch constants"));
     const int64_t total_words = P.word_prefix[E];
     uint32_t* bits = static_cast<uint32_t*>(W.bits.ensure(
-        (size_t)(total_words + 16) * 4 + (size_t)kFlagListCap * 8, "batch flag bitmaps and queue"));
+        (size_t)(total_words + 16) * 4 + (size_t)kFlagListCap * 8 + 16, "batch flag bitmaps and queue"));
 
     std::vector<BatchEns> ens(E);
     for (int e = 0; e < E; ++e) {
@@ -371,6 +370,8 @@ void enqueue(bs_context* ctx, const Plan& P, const std::vector<const double*>& d
     a.ens_bits0 = bits;
     a.counters = bits + total_words;
     a.flag_list = reinterpret_cast<int64_t*>(bits + total_words + 16);
+    a.t_start = reinterpret_cast<uint64_t*>(a.flag_list + kFlagListCap);
+    a.clocks = ctx->batch_clocks();
     a.n_wg = std::max(1, std::min(2 * ctx->n_cu, (int)P.items.size()));
 
     // graph of this shape: the kernel arguments are all that it bakes in
@@ -401,13 +402,10 @@ void enqueue(bs_context* ctx, const Plan& P, const std::vector<const double*>& d
         ++W.graph_builds;
     }
     // the stages run inside the graph: only the total is timed
-    rec->mark({kBTotal0, kBPrep0, kBPrep1, kBMain0, kBMain1, kBFallback0, kBFallback1}, s);
     BS_HIP(hipGraphLaunch(W.exec, s));
-    rec->mark({kBTotal1}, s);
     ++W.graph_launches;
-    if (rec->h_count)
-        BS_HIP(hipMemcpyAsync(rec->h_count, a.counters + kLists, 4, hipMemcpyDeviceToHost, s));
-    rec->gram = true;
+    rec->clk = ctx->batch_clocks() + kClkWords * (1 + ctx->batch_replays++ % kBatchClocks);
+    rec->kind = RunRecord::kTotalOnly;
     rec->base.tile_m = rec->base.tile_n = P.tile.empty() ? 0 : P.tile[0];
 }
 

@@ -51,21 +51,23 @@ static PrepView prep_view(const PreparedPtrs& p, const double* d_xyz, int n, int
 }
 
 PrepView prepare_into(const PreparedPtrs& p, const double* d_xyz, int n, int L, GramMode mode,
-                      const double* fixed_ref, hipStream_t s)
+                      const double* fixed_ref, hipStream_t s, uint64_t* t_start)
 {
     const int n_pad = round_up(n, kTileRows), n_kblk = (L + kAtomBlock - 1) / kAtomBlock;
     const double* ref = fixed_ref;  // a fixed reference is read in place
     if (!fixed_ref) {
-        launch_reference(d_xyz, n, L, p.partial, p.ref, s);
+        launch_reference(d_xyz, n, L, p.partial, p.ref, s, t_start);
+        t_start = nullptr;
         ref = p.ref;
     }
-    launch_fit_pack(d_xyz, ref, n, n_pad, L, n_kblk, mode, p.rot, p.cent, p.panels, p.consts, n_pad, s);
+    launch_fit_pack(d_xyz, ref, n, n_pad, L, n_kblk, mode, p.rot, p.cent, p.panels, p.consts, n_pad, s,
+                    t_start);
     BS_HIP(hipGetLastError());
     return prep_view(p, d_xyz, n, L, mode);
 }
 
 void prepare(Prepared& P, const double* d_xyz, int n, int L, GramMode mode,
-             const double* fixed_ref, hipStream_t s)
+             const double* fixed_ref, hipStream_t s, uint64_t* t_start)
 {
     P.n = n;
     P.L = L;
@@ -83,7 +85,7 @@ void prepare(Prepared& P, const double* d_xyz, int n, int L, GramMode mode,
         p.ref = static_cast<double*>(P.ref.ensure(z.ref, "reference"));
         p.partial = static_cast<double*>(P.partial.ensure(z.partial, "reference partial sums"));
     }
-    (void)prepare_into(p, d_xyz, n, L, mode, fixed_ref, s);
+    (void)prepare_into(p, d_xyz, n, L, mode, fixed_ref, s, t_start);
 }
 
 GramThresholds gram_thresholds(GramMode mode, int L, int n_kblk)
@@ -124,48 +126,23 @@ EpilogueLimits epilogue_limits(const GramThresholds& t, int L)
     return e;
 }
 
-void RunRecord::create()
-{
-    for (auto& e : ev) BS_HIP(hipEventCreate(&e));
-}
-
-void RunRecord::destroy()
-{
-    for (auto& e : ev)
-        if (e) (void)hipEventDestroy(e);
-}
-
-void RunRecord::reset()
-{
-    for (auto& x : slot) x = -1;
-    n_ev = 0;
-}
-
-void RunRecord::mark(std::initializer_list<int> bounds, hipStream_t s)
-{
-    BS_REQUIRE(n_ev < 8, "too many events in one run record");
-    BS_HIP(hipEventRecord(ev[n_ev], s));
-    for (int b : bounds) slot[b] = (int8_t)n_ev;
-    ++n_ev;
-}
-
 bs_run_stats RunRecord::read() const
 {
     bs_run_stats st = base;
-    if (!used || n_ev == 0) return st;
-    BS_HIP(hipEventSynchronize(ev[n_ev - 1]));
-    auto span = [&](int k) {
-        const int a = slot[2 * k], b = slot[2 * k + 1];
-        if (a < 0 || b < 0 || a == b) return 0.0;
-        float v = 0.0f;
-        BS_HIP(hipEventElapsedTime(&v, ev[a], ev[b]));
-        return (double)v;
-    };
-    st.total_ms = span(kRecTotal);
-    st.prep_ms = span(kRecPrep);
-    st.main_ms = span(kRecMain);
-    st.fallback_ms = span(kRecFallback);
-    st.flagged_pairs = gram && h_count ? *h_count : base.flagged_pairs;
+    if (kind == kUntimed) return st;
+    uint64_t t[kClkWords];
+    BS_HIP(hipStreamSynchronize(stream));
+    BS_HIP(hipMemcpy(t, clk, sizeof(t), hipMemcpyDeviceToHost));
+    auto ms = [&](int a, int b) { return t[b] > t[a] ? (double)(t[b] - t[a]) / khz : 0.0; };
+    st.total_ms = ms(kClkStart, kClkEnd);
+    if (kind == kOneStage) st.main_ms = st.total_ms;
+    if (kind == kTwoStages || kind == kAllStages) st.prep_ms = ms(kClkStart, kClkMain);
+    if (kind == kTwoStages) st.main_ms = ms(kClkMain, kClkEnd);
+    if (kind == kAllStages) {
+        st.main_ms = ms(kClkMain, kClkResolve);
+        st.fallback_ms = ms(kClkResolve, kClkResolveEnd);
+    }
+    if (kind == kAllStages || kind == kTotalOnly) st.flagged_pairs = t[kClkCount];
     return st;
 }
 
@@ -187,8 +164,7 @@ PrepView view_of(const Prepared& P, int first, int count)
 }
 
 void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, const uint32_t* order,
-                   int n_tiles, uint32_t* flags, int list_cap, bool clear_flags, int max_wg, hipStream_t s,
-                   RunRecord* rec)
+                   int n_tiles, uint32_t* flags, int list_cap, bool clear_flags, int max_wg, hipStream_t s)
 {
     // Flagged outputs go to a list of list_cap positions (counted in the
     // control words at the region's start); any beyond it set bits of a
@@ -197,7 +173,6 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     // kernel then re-evaluates them in FP64 and leaves the region clean.
     const uint64_t n_out =
         run.triangle ? (uint64_t)A.n * (A.n - 1) / 2 : (uint64_t)A.n * (uint64_t)run.out_ld;
-    const uint64_t n_words = flag_words(n_out);
     uint32_t* ctl = flags;  // count, report, done, spare
     int64_t* list = reinterpret_cast<int64_t*>(flags + 4);
     uint32_t* bits = reinterpret_cast<uint32_t*>(list + list_cap);
@@ -231,31 +206,23 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
                "row statistics need the f32 triangle");
     g.stats_part = run.stats_part;
     g.stats_T = (A.n + kTileRows - 1) / kTileRows;
-    (void)n_words;
+    g.t_start = run.clk && run.clk_main ? run.clk + kClkMain : nullptr;
 
-    if (rec) rec->mark({kBPrep1, kBMain0}, s);
     launch_gram(g, A.mode, s);
-    if (rec) rec->mark({kBMain1, kBFallback0}, s);
     BS_HIP(hipGetLastError());
     // the statistics of the pairs the epilogue kept, as keys; the resolve
     // kernel then adds the re-evaluated pairs, and the keys become f32
     if (stats) launch_row_stats_combine(run.stats_part, A.n, run.st_min, run.st_max, s);
     launch_flag_resolve(A.xyz, A.cent, B.xyz, B.cent, A.L, ctl, list, list_cap, bits, (int64_t)n_out,
-                        g.triangle, A.n, run.out_ld, run.d_out, g.out_f64, rec ? rec->h_count : nullptr,
-                        run.h_count, run.st_min, run.st_max, s);
-    if (stats) launch_row_stats_decode(run.st_min, run.st_max, A.n, s);
+                        g.triangle, A.n, run.out_ld, run.d_out, g.out_f64, run.h_count, run.st_min,
+                        run.st_max, run.clk_resolve ? run.clk : nullptr, run.ends_call && !stats, s);
+    if (stats)
+        launch_row_stats_decode(run.st_min, run.st_max, A.n, s, run.clk ? run.clk + kClkEnd : nullptr, run.done);
     BS_HIP(hipGetLastError());
-    if (rec) {
-        if (run.ends_total)
-            rec->mark({kBFallback1, kBTotal1}, s);
-        else
-            rec->mark({kBFallback1}, s);
-        rec->gram = true;
-    }
 }
 
 void run_gram(const PrepView& A, const PrepView& B, const GramRun& run, GramScratch& sc,
-              hipStream_t s, RunRecord* rec)
+              hipStream_t s)
 {
     BS_REQUIRE(A.L == B.L && A.mode == B.mode, "prepared sets disagree on atom count or mode");
     const int tiles_r = (A.n + kTileRows - 1) / kTileRows, tiles_c = (B.n + kTileRows - 1) / kTileRows;
@@ -271,7 +238,7 @@ void run_gram(const PrepView& A, const PrepView& B, const GramRun& run, GramScra
     if (sc.flags_clean != sc.flags.generation())
         launch_zero_words(flags, (int64_t)(sc.flags.size() / 16 * 4), s);
     sc.flags_clean = 0;  // a sequence that throws part-way leaves the region unknown
-    run_gram_with(A, B, run, order, n_tiles, flags, kFlagListCap, false, sc.max_wg, s, rec);
+    run_gram_with(A, B, run, order, n_tiles, flags, kFlagListCap, false, sc.max_wg, s);
     sc.flags_clean = sc.flags.generation();
 }
 
@@ -352,31 +319,29 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
     RunRecord* rec = ctx->begin_record();
     rec->base.pairs = n >= 2 ? (uint64_t)n * (n - 1) / 2 : 0;
     if (n >= 2 && !is_gram(m)) {
-        rec->mark({kBTotal0, kBPrep0, kBPrep1, kBMain0}, s);
-        launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s);
+        launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s, rec->clk, rec->done);
         BS_HIP(hipGetLastError());
-        rec->mark({kBMain1, kBFallback0, kBFallback1, kBTotal1}, s);
+        rec->kind = RunRecord::kOneStage;
         rec->base.main_launches = 1;
     } else if (n >= 2) {
-        rec->mark({kBTotal0, kBPrep0}, s);
-        prepare(ctx->prep, d_xyz, n, L, mode_of(m), nullptr, s);
+        prepare(ctx->prep, d_xyz, n, L, mode_of(m), nullptr, s, rec->clk + kClkStart);
         GramRun run;
         run.triangle = true;
         run.d_out = d_out;
         run.out_f64 = out_f64;
-        run.ends_total = true;
+        run.clk = rec->clk;
+        run.done = rec->done;
         if (fused) {
             run.stats_part = static_cast<unsigned*>(
                 ctx->ws_stats.ensure(fused_stats_tiles(n) * 256 * 4, "row statistics tiles"));
             run.st_min = reinterpret_cast<unsigned*>(d_rmin);
             run.st_max = reinterpret_cast<unsigned*>(d_rmax);
         }
-        run_gram(view_of(ctx->prep), view_of(ctx->prep), run, ctx->gsc, s, rec);
+        run_gram(view_of(ctx->prep), view_of(ctx->prep), run, ctx->gsc, s);
+        rec->kind = RunRecord::kAllStages;
         rec->base.main_launches = 1;
         rec->base.tile_m = kTileRows;
         rec->base.tile_n = kTileRows;
-    } else {
-        rec->mark({kBTotal0, kBTotal1, kBPrep0, kBPrep1, kBMain0, kBMain1, kBFallback0, kBFallback1}, s);
     }
     if (d_rmin && !fused) {
         void* scratch = ctx->ws_stats.ensure(row_stats_scratch_bytes(n), "row statistics tiles");
@@ -389,20 +354,23 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
 
 bs::RunRecord* bs_context::begin_record()
 {
-    constexpr size_t kRing = 64;
     if (ring.empty()) {
+        const size_t words = (kRing + 1 + bs::kBatchClocks + 1) * bs::kClkWords;
+        auto* clk = static_cast<uint64_t*>(ws_clock.ensure(words * 8, "call clocks"));
+        bs::launch_zero_u32(reinterpret_cast<uint32_t*>(clk), (int)(2 * words), stream);
+        BS_HIP(hipGetLastError());
         ring.resize(kRing);
-        for (auto& r : ring) r.create();
-        BS_HIP(hipHostMalloc((void**)&h_counts, kRing * sizeof(uint32_t), hipHostMallocDefault));
-        for (size_t k = 0; k < kRing; ++k) ring[k].h_count = h_counts + k;
+        for (auto& r : ring) {
+            r.done = reinterpret_cast<unsigned*>(clk + words - bs::kClkWords);
+            r.stream = stream;
+            r.khz = clock_khz;
+        }
     }
     bs::RunRecord* r = &ring[ring_next];
+    r->clk = ws_clock.as<uint64_t>() + ring_next * bs::kClkWords;
     ring_next = (ring_next + 1) % ring.size();
     ring_used = std::min(ring_used + 1, ring.size());
-    if (r->used && r->n_ev > 0) BS_HIP(hipEventSynchronize(r->ev[r->n_ev - 1]));  // never reuse in flight
-    r->reset();
+    r->kind = bs::RunRecord::kUntimed;
     r->base = bs_run_stats{};
-    r->gram = false;
-    r->used = true;
     return r;
 }

@@ -84,11 +84,12 @@ PreparedSizes prepared_sizes(int n, int L);
 // onto it, read in place (Prepared::ref stays unused); otherwise the reference
 // is one Procrustes-mean step from conformation 0 over the reference samples.
 // d_xyz is borrowed (Prepared::xyz).
+// t_start: clock word of the first launch's start, or null.
 void prepare(Prepared& P, const double* d_xyz, int n, int L, GramMode mode,
-             const double* fixed_ref, hipStream_t s);
+             const double* fixed_ref, hipStream_t s, uint64_t* t_start = nullptr);
 // The same into caller-provided buffers; returns the view the Gram run reads.
 PrepView prepare_into(const PreparedPtrs& p, const double* d_xyz, int n, int L, GramMode mode,
-                      const double* fixed_ref, hipStream_t s);
+                      const double* fixed_ref, hipStream_t s, uint64_t* t_start = nullptr);
 
 // Flagging thresholds of the Gram epilogue's error model at atom count L.
 struct GramThresholds {
@@ -100,11 +101,15 @@ EpilogueLimits epilogue_limits(const GramThresholds& t, int L);
 
 struct GramRun {
     uint32_t* h_count = nullptr;  // pinned: receives the flagged-pair count (async)
+    // the call's clock (stamp.hpp): whether the Gram launch's start, the
+    // re-evaluation's times and the call's end are taken in this run
+    uint64_t* clk = nullptr;
+    bool clk_main = true, clk_resolve = true, ends_call = true;
+    unsigned* done = nullptr;     // zero device word (with row statistics)
     bool triangle = true;
     void* d_out = nullptr;
     bool out_f64 = false;
     int64_t out_ld = 0;
-    bool ends_total = false;      // the record's total ends with this run
     // row statistics from the epilogue (triangle, f32 output): tile results
     // (fused_stats_tiles(n) x 1 KiB) and the n keys of each statistic, which
     // the run leaves decoded to f32
@@ -147,35 +152,25 @@ struct GramScratch {
     static size_t order_bytes(size_t max_tiles) { return kOrders * (max_tiles * 4 + 4); }
 };
 
-// Events and host-visible results of one call, read lazily.
-// Stage boundaries of a call's record: 2k starts stage k, 2k + 1 ends it.
-enum { kRecTotal = 0, kRecPrep = 1, kRecMain = 2, kRecFallback = 3 };
-enum {
-    kBTotal0 = 0, kBTotal1 = 1, kBPrep0 = 2, kBPrep1 = 3,
-    kBMain0 = 4, kBMain1 = 5, kBFallback0 = 6, kBFallback1 = 7
-};
-
-// Timing of one call.  Each mark() records one event for the boundaries it
-// names, so boundaries with no work between them share an event: an event
-// record costs the stream a few microseconds, as much as a small kernel.
+// Times and flagged count of one call, taken by its own kernels (stamp.hpp)
+// and read on demand.  Calls of a context follow each other on its stream, so
+// a record's words are reused without waiting.
 struct RunRecord {
-    hipEvent_t ev[8] = {};        // in the order recorded
-    int8_t slot[8] = {-1, -1, -1, -1, -1, -1, -1, -1};  // boundary -> index into ev
-    int n_ev = 0;
-    uint32_t* h_count = nullptr;  // flagged-pair count (pinned), stored by the resolve kernel
+    // which words the call stores: none; start, end (the per-pair kernels);
+    // start, end, count (a batch: its stages run inside a graph); start, main,
+    // end (streamed blocks); all of them
+    enum Kind { kUntimed, kOneStage, kTotalOnly, kTwoStages, kAllStages };
+    uint64_t* clk = nullptr;      // kClkWords device words
+    unsigned* done = nullptr;     // zero device word for the last launch's stamp
+    hipStream_t stream = nullptr;
+    int khz = 0;                  // the clock's rate
+    Kind kind = kUntimed;
     bs_run_stats base{};          // pairs, launches, tile sizes
-    bool gram = false;
-    bool used = false;
-    void create();
-    void destroy();
-    void reset();
-    void mark(std::initializer_list<int> bounds, hipStream_t s);
-    bs_run_stats read() const;  // synchronises on the last event
+    bs_run_stats read() const;    // waits for the stream
 };
 
 // Gram contraction + QCP epilogue + FP64 re-evaluation of flagged pairs over
-// rows of A x cols of B (or the upper triangle of A when triangle).  Asynchronous:
-// the flagged-pair count is stored to rec->h_count when rec is given.
+// rows of A x cols of B (or the upper triangle of A when triangle).  Asynchronous.
 // Words of the flag bitmap of n_out outputs (a whole number of 16-byte units).
 inline uint64_t flag_words(uint64_t n_out) { return ((n_out + 31) / 32 + 3) / 4 * 4; }
 // Bytes of the flag region: four control words (count, report, done, spare),
@@ -188,14 +183,13 @@ inline size_t flag_region_bytes(uint64_t n_out, int list_cap)
 }
 // The Gram launch sequence with every buffer given: `order` (n_tiles tile
 // codes on the device), `flags` (flag_region_bytes(n_out, list_cap)); no
-// allocation, no host copy except the optional counts of `run` / `rec`.
+// allocation, no host copy.
 // Each launch leaves the region's control words zero and its bitmap clear;
 // `clear_flags` zeroes the region first, for memory that may hold anything.
 void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, const uint32_t* order,
-                   int n_tiles, uint32_t* flags, int list_cap, bool clear_flags, int max_wg, hipStream_t s,
-                   RunRecord* rec);
+                   int n_tiles, uint32_t* flags, int list_cap, bool clear_flags, int max_wg, hipStream_t s);
 void run_gram(const PrepView& A, const PrepView& B, const GramRun& run, GramScratch& sc,
-              hipStream_t s, RunRecord* rec);
+              hipStream_t s);
 
 // Workspace of one in-flight query batch (query prep, score matrix, top-k).
 struct QueryWorkspace {
@@ -248,7 +242,12 @@ struct bs_context {
     bs::QueryWorkspace qws;    // synchronous query calls
     std::vector<bs::RunRecord> ring;  // the last calls' records
     size_t ring_next = 0, ring_used = 0;
-    uint32_t* h_counts = nullptr;      // pinned, one per record
+    // clocks: kClkWords per record, those of the batch graphs (which write to
+    // the clock of their replay, not of a record), the calls' zero word
+    bs::DevBuf ws_clock;
+    uint64_t batch_replays = 0;        // batch graphs launched, as the device counts them
+    uint64_t* batch_clocks() { return ws_clock.as<uint64_t>() + kRing * bs::kClkWords; }
+    static constexpr size_t kRing = 64;
     bs::RunRecord* begin_record();     // next ring slot, recycled
     std::vector<bs::TuneCell> tune[4];  // autotuner: Gram tile side per (L, n) cell, per method
     bs::BatchWorkspace batch;          // batched pipeline (bs_crmsd_batch*)

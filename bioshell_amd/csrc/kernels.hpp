@@ -6,6 +6,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "stamp.hpp"
+
 namespace bs {
 
 // ------------------------------------------------------------ plain path
@@ -16,8 +18,10 @@ namespace bs {
 // (fp64), chosen by plain_block from the pair slots the tiles cover and, for
 // a lone launch (alone), from how many rounds of 2 work-groups per CU they
 // take on n_cu CUs.
+// clk (a call's clock, stamp.hpp) gets the launch's start and end; done is its
+// zero word.
 void launch_plain_avsa(const double* xyz, int n, int L, bool fp64, void* out, bool out_f64,
-                       int n_cu, hipStream_t s);
+                       int n_cu, hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
 int plain_block(int n, bool fp64, bool alone, int n_cu);
 inline int plain_tiles_per_side(int n, int r) { return (n + 16 * r - 1) / (16 * r); }
 // One ensemble of a batched plain launch (f32 output); nt tiles per side.
@@ -29,7 +33,7 @@ struct PlainEns {
 // Every ensemble of ens[0 .. n_ens) with block r in one launch: prefix (n_ens + 1
 // entries, device) counts their tiles, tiles = prefix[n_ens].
 void launch_plain_batch(const PlainEns* ens, const int* prefix, int n_ens, int tiles, int r, bool fp64,
-                        hipStream_t s);
+                        hipStream_t s, uint64_t* t_start, uint64_t* t_end, unsigned* done);
 
 // ------------------------------------------------------------ Gram path
 enum GramMode : int { kGramBF16x3 = 0, kGramFP32 = 1 };
@@ -79,12 +83,13 @@ __host__ __device__ inline int ref_sample_index(int s, int n, int S)
 // Reference of one ensemble (prep_device.hpp): for the S = ref_sample_count(n)
 // samples, the slices' partial sums of the fitted samples (partial,
 // ref_slices(S) x 3L), then r (ref: 3L values) and R0 (6).
-void launch_reference(const double* xyz, int n, int L, double* partial, double* ref, hipStream_t s);
+void launch_reference(const double* xyz, int n, int L, double* partial, double* ref, hipStream_t s,
+                      uint64_t* t_start);
 // Fit onto ref and pack: rotations (rot), centroids (cent), operand panels of
 // e_i = rot_i (x_i - c_i) - ref and the constants, for n_pad rows.
 void launch_fit_pack(const double* xyz, const double* ref, int n, int n_pad, int L, int n_kblk,
                      GramMode mode, double* rot, double* cent, void* panels, double* consts, int ld,
-                     hipStream_t s);
+                     hipStream_t s, uint64_t* t_start);
 
 // The epilogue's flagging limits and RMSD scale at one atom count L, formed
 // on the host so that the kernels hold them in scalar registers rather than
@@ -129,6 +134,7 @@ struct GramArgs {
     // the flagged pairs (the resolve kernel adds their final values).
     unsigned* stats_part;
     int stats_T;            // tiles per side of the triangle
+    uint64_t* t_start;      // clock word of the launch's start, or null
 };
 
 // Builds the logical tile order (XCD-aware super-blocks) on the host.
@@ -144,16 +150,18 @@ void launch_zero_u32(uint32_t* p, int n, hipStream_t s);
 // bitmap `bits` (n_out bits) that clears every word it reads.  ctl holds
 // count, report, done: the last work-group to finish copies count to report
 // and zeroes count and done, so the region is ready for the next launch.  It
-// also stores the count into h_report_a / h_report_b when given (pinned host
-// words, written with a system-scope store: no separate device-to-host copy).
+// also stores the count into h_report when given (a pinned host word, written
+// with a system-scope store: no separate device-to-host copy).  clk (a call's
+// clock, or null) gets the launch's start and end, the count and, with
+// ends_call, the call's end.
 // With st_min / st_max set (triangle, f32 output), each re-evaluated value
 // also goes into the row-statistics keys of both its elements (atomic
 // min / max on order-preserving keys).
 void launch_flag_resolve(const double* xyz_a, const double* cent_a, const double* xyz_b,
                          const double* cent_b, int L, uint32_t* ctl, const int64_t* list, int cap,
                          uint32_t* bits, int64_t n_out, int triangle, int n, int64_t out_ld, void* out,
-                         int out_f64, uint32_t* h_report_a, uint32_t* h_report_b, unsigned* st_min,
-                         unsigned* st_max, hipStream_t s);
+                         int out_f64, uint32_t* h_report, unsigned* st_min, unsigned* st_max,
+                         uint64_t* clk, bool ends_call, hipStream_t s);
 // Queues the set bits of bits[0 .. n_words) as bit indices (word * 32 + bit)
 // into list (cap entries), clearing the queued ones; *count += set bits.
 void launch_flag_compact(uint32_t* bits, int64_t n_words, int64_t* list, int cap, uint32_t* count,
@@ -171,7 +179,7 @@ size_t topk_scratch_bytes(int n_q, int n_lib, int k);
 // k for a given n_lib.
 bool topk_supported(int n_lib, int k);
 void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, float* val, void* scratch,
-                 hipStream_t s);
+                 hipStream_t s, uint64_t* t_end = nullptr, unsigned* done = nullptr);
 
 // ------------------------------------------------------------ batches
 // One ensemble of a batch, as the batched kernels see it (device memory).
@@ -202,6 +210,7 @@ struct BatchEns {
 // tile (bit 31 clear: index into tiles64) or four 32 x 32 tiles, one per
 // wave (bit 31 set: index q, tiles32[4q .. 4q+3]).  Tile codes are
 // (ensemble << 32) | (tile row << 16) | tile col; ~0 marks an empty slot.
+constexpr int kBatchClocks = 64;  // clocks of the last replays of batch graphs
 struct BatchArgs {
     const BatchEns* ens;
     int n_ens;
@@ -220,6 +229,8 @@ struct BatchArgs {
     uint32_t* counters;     // 8 list counters, then the flagged-pair count
     int64_t* flag_list;     // kFlagListCap queued re-evaluations (batch-wide bit indices)
     int n_wg;               // persistent work-groups of the Gram kernel
+    uint64_t* t_start;      // device word: the clock at the batch's start
+    uint64_t* clocks;       // replay counter (kClkWords words), then kBatchClocks clocks
 };
 
 // The batched pipeline's launches, in order (each over all ensembles).
@@ -253,7 +264,8 @@ inline size_t fused_stats_tiles(int n)
 // Combines the epilogue's tile results into keys (kmin / kmax, n each, n >= 2),
 // which the resolve kernel then updates; decode turns the keys into f32.
 void launch_row_stats_combine(const unsigned* part, int n, unsigned* kmin, unsigned* kmax, hipStream_t s);
-void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s);
+void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end,
+                             unsigned* done);
 // For each of m members, the largest distance to the other members.
 void launch_members_row_max(const float* up, int n, const unsigned* members, int m, float* out,
                             hipStream_t s);

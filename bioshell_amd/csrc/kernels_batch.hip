@@ -37,6 +37,7 @@ __device__ inline int find_ens(const T* __restrict__ prefix, int n_ens, T g)
 __global__ __launch_bounds__(256) void batch_fit0_kernel(BatchArgs b)
 {
     __shared__ Fit0Lds lds;
+    stamp_start(b.t_start);
     const int g = blockIdx.x;
     const int e = find_ens(b.slice_prefix, b.n_ens, g);
     const BatchEns& E = b.ens[e];
@@ -227,6 +228,19 @@ __global__ __launch_bounds__(256) void batch_fallback_kernel(BatchArgs b)
     }
 }
 
+// The graph's last node: the start word, the time this kernel starts and the
+// count of flagged pairs go to the clock of this replay, which the replay
+// counter selects (the host counts replays too).
+__global__ void batch_report_kernel(BatchArgs b)
+{
+    const uint64_t k = b.clocks[0];
+    uint64_t* clk = b.clocks + kClkWords * (1 + k % kBatchClocks);
+    clk[kClkEnd] = wall_clock64();
+    clk[kClkStart] = *b.t_start;
+    clk[kClkCount] = b.counters[kXcd];
+    b.clocks[0] = k + 1;
+}
+
 }  // namespace
 
 void launch_batch_prep(const BatchArgs& b, hipStream_t s)
@@ -260,6 +274,7 @@ void launch_batch_fallback(const BatchArgs& b, hipStream_t s)
     const int64_t waves = (b.total_words + 63) / 64;
     const int64_t blocks = std::min<int64_t>(2048, std::max<int64_t>(1, (waves + 3) / 4));
     batch_fallback_kernel<<<(int)blocks, 256, 0, s>>>(b);
+    batch_report_kernel<<<1, 1, 0, s>>>(b);
 }
 
 }  // namespace bs

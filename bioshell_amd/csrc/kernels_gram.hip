@@ -35,6 +35,7 @@ template <int MODE, bool STATS>
 __global__ __launch_bounds__(256, 2) void gram_kernel(GramArgs a)
 {
     __shared__ uint4 lds[3][4][kPanelBlockU4];  // 3 stages x (A0, A1, B0, B1) x 6 KiB
+    stamp_start(a.t_start);
     const int wg = blockIdx.x;
     const int per = (a.n_tiles + kXcd - 1) / kXcd;
     const int t = (wg % kXcd) * per + (wg / kXcd);
@@ -155,9 +156,10 @@ __global__ __launch_bounds__(256) void flag_resolve_kernel(const double* __restr
                                                            uint32_t* __restrict__ bits, int64_t n_out,
                                                            int triangle, int n, int64_t out_ld,
                                                            void* __restrict__ out, int out_f64,
-                                                           uint32_t* h_report_a, uint32_t* h_report_b,
-                                                           unsigned* st_min, unsigned* st_max)
+                                                           uint32_t* h_report, unsigned* st_min,
+                                                           unsigned* st_max, uint64_t* clk, int ends_call)
 {
+    stamp_start(clk ? clk + kClkResolve : nullptr);
     const int lane = threadIdx.x & 63;
     const uint32_t cnt = ctl[0];  // read before this group counts itself done
     const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -194,8 +196,13 @@ __global__ __launch_bounds__(256) void flag_resolve_kernel(const double* __restr
         ctl[1] = cnt;
         ctl[0] = 0u;
         ctl[2] = 0u;
-        if (h_report_a) __hip_atomic_store(h_report_a, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (h_report_b) __hip_atomic_store(h_report_b, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (h_report) __hip_atomic_store(h_report, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (clk) {
+            const uint64_t now = wall_clock64();
+            clk[kClkResolveEnd] = now;
+            clk[kClkCount] = cnt;
+            if (ends_call) clk[kClkEnd] = now;
+        }
     }
 }
 
@@ -245,8 +252,8 @@ void launch_zero_words(uint32_t* p, int64_t n_words, hipStream_t s)
 void launch_flag_resolve(const double* xyz_a, const double* cent_a, const double* xyz_b,
                          const double* cent_b, int L, uint32_t* ctl, const int64_t* list, int cap,
                          uint32_t* bits, int64_t n_out, int triangle, int n, int64_t out_ld, void* out,
-                         int out_f64, uint32_t* h_report_a, uint32_t* h_report_b, unsigned* st_min,
-                         unsigned* st_max, hipStream_t s)
+                         int out_f64, uint32_t* h_report, unsigned* st_min, unsigned* st_max,
+                         uint64_t* clk, bool ends_call, hipStream_t s)
 {
     // 1024 waves: a typical list (tens to thousands of pairs) is one pass, a
     // full list or a bitmap scan takes several.  A grid sized for the bitmap
@@ -254,7 +261,7 @@ void launch_flag_resolve(const double* xyz_a, const double* cent_a, const double
     // done-counter atomics of the idle groups.
     flag_resolve_kernel<<<256, 256, 0, s>>>(
         xyz_a, cent_a, xyz_b, cent_b, L, ctl, list, cap, bits, n_out, triangle, n, out_ld, out, out_f64,
-        h_report_a, h_report_b, st_min, st_max);
+        h_report, st_min, st_max, clk, ends_call ? 1 : 0);
 }
 
 void launch_flag_compact(uint32_t* bits, int64_t n_words, int64_t* list, int cap, uint32_t* count,

@@ -11,9 +11,10 @@ namespace {
 // the mean (thread per coordinate, one wave per work-group to spread the few
 // coordinates over more CUs), then R0 (one block).
 __global__ __launch_bounds__(256) void fit0_kernel(const double* __restrict__ xyz, int n, int S,
-                                                   int L, double* __restrict__ partial)
+                                                   int L, double* __restrict__ partial, uint64_t* t_start)
 {
     __shared__ Fit0Lds lds;
+    stamp_start(t_start);
     fit0_slice(xyz, n, S, L, blockIdx.x, partial, lds);
 }
 
@@ -39,9 +40,11 @@ __global__ __launch_bounds__(256) void fit_pack_kernel(const double* __restrict_
                                                        double* __restrict__ rot,
                                                        double* __restrict__ cent,
                                                        uint4* __restrict__ panels,
-                                                       double* __restrict__ consts, int ld)
+                                                       double* __restrict__ consts, int ld,
+                                                       uint64_t* t_start)
 {
     __shared__ FitPackLds lds;
+    stamp_start(t_start);
     const int blk = xcd_contiguous_block(fit_groups(n_pad));
     if (blk < 0) return;
     fit_pack_block<MODE>(xyz, ref, n, L, n_kblk, blk * kFitConfs, rot, cent, panels, consts, ld, lds);
@@ -92,27 +95,28 @@ __global__ __launch_bounds__(64) void superpose_kernel(const double* __restrict_
 
 }  // namespace
 
-void launch_reference(const double* xyz, int n, int L, double* partial, double* ref, hipStream_t s)
+void launch_reference(const double* xyz, int n, int L, double* partial, double* ref, hipStream_t s,
+                      uint64_t* t_start)
 {
     const int S = ref_sample_count(n);
     const int slices = ref_slices(S);
-    fit0_kernel<<<slices, 256, 0, s>>>(xyz, n, S, L, partial);
+    fit0_kernel<<<slices, 256, 0, s>>>(xyz, n, S, L, partial, t_start);
     mean_final_kernel<<<(3 * L + 63) / 64, 64, 0, s>>>(partial, slices, S, L, ref);
     ref_gram_kernel<<<1, 256, 0, s>>>(ref, L);
 }
 
 void launch_fit_pack(const double* xyz, const double* ref, int n, int n_pad, int L, int n_kblk,
                      GramMode mode, double* rot, double* cent, void* panels, double* consts, int ld,
-                     hipStream_t s)
+                     hipStream_t s, uint64_t* t_start)
 {
     const int blocks = xcd_contiguous_grid(fit_groups(n_pad));
     uint4* p = static_cast<uint4*>(panels);
     if (mode == kGramBF16x3)
         fit_pack_kernel<kGramBF16x3><<<blocks, 256, 0, s>>>(xyz, ref, n, n_pad, L, n_kblk, rot,
-                                                            cent, p, consts, ld);
+                                                            cent, p, consts, ld, t_start);
     else
         fit_pack_kernel<kGramFP32><<<blocks, 256, 0, s>>>(xyz, ref, n, n_pad, L, n_kblk, rot, cent,
-                                                          p, consts, ld);
+                                                          p, consts, ld, t_start);
 }
 
 void launch_superpose(const double* a, const double* b, int L, double* out13, hipStream_t s)

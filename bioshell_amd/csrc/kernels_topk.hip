@@ -170,7 +170,8 @@ __global__ __launch_bounds__(kChunkThreads) void topk_chunk_kernel(const float* 
 
 __global__ __launch_bounds__(1024) void topk_merge_kernel(const unsigned long long* __restrict__ cand, int m,
                                                           int k, uint32_t* __restrict__ out_idx,
-                                                          float* __restrict__ out_val)
+                                                          float* __restrict__ out_val, uint64_t* t_end,
+                                                          unsigned* done)
 {
     __shared__ unsigned long long s[kMergeMax];
     const int q = blockIdx.x, tid = threadIdx.x;
@@ -199,6 +200,7 @@ __global__ __launch_bounds__(1024) void topk_merge_kernel(const unsigned long lo
         out_idx[(int64_t)q * k + v] = (uint32_t)(c & 0xFFFFFFFFu);
         out_val[(int64_t)q * k + v] = __uint_as_float((uint32_t)(c >> 32));
     }
+    stamp_end(t_end, done);
 }
 
 // Chunk length: at least kMinChunk, a multiple of 256, and few enough chunks
@@ -230,7 +232,7 @@ bool topk_supported(int n_lib, int k)
 }
 
 void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, float* val, void* scratch,
-                 hipStream_t s)
+                 hipStream_t s, uint64_t* t_end, unsigned* done)
 {
     if (n_q <= 0) return;
     if (k <= 0 || k > kTopkMax || k > n_lib) fail(BS_ERR_INVALID_ARGUMENT, "top-k: k = %d outside [1, min(%d, %d)]",
@@ -241,7 +243,7 @@ void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, 
     const int n_chunks = (n_lib + chunk - 1) / chunk;
     auto* cand = static_cast<unsigned long long*>(scratch);
     topk_chunk_kernel<<<dim3(n_chunks, n_q), kChunkThreads, 0, s>>>(scores, n_lib, k, chunk, cand);
-    topk_merge_kernel<<<n_q, 1024, 0, s>>>(cand, n_chunks * k, k, idx, val);
+    topk_merge_kernel<<<n_q, 1024, 0, s>>>(cand, n_chunks * k, k, idx, val, t_end, done);
 }
 
 }  // namespace bs

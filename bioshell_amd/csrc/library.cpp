@@ -77,23 +77,27 @@ void enqueue_query(bs_library* lib, QueryWorkspace& ws, const double* q_host, in
     float* scores =
         static_cast<float*>(ws.scores.ensure((size_t)n_q * n_lib * 4, "query scores"));
     BS_HIP(hipMemcpyAsync(dq, q_host, (size_t)n_q * L * 3 * 8, hipMemcpyHostToDevice, s));
-    if (rec) rec->mark({kBTotal0, kBPrep0}, s);
-    prepare(ws.prep, dq, n_q, L, lib->P.mode, lib->P.ref.as<double>(), s);
+    prepare(ws.prep, dq, n_q, L, lib->P.mode, lib->P.ref.as<double>(), s, rec ? rec->clk + kClkStart : nullptr);
     GramRun run;
+    if (rec) {
+        run.clk = rec->clk;
+        run.ends_call = k == 0;
+    }
     run.triangle = false;
     run.d_out = scores;
     run.out_f64 = false;
     run.out_ld = n_lib;
     ws.gsc.max_wg = lib->ctx->gsc.max_wg;
-    run_gram(view_of(ws.prep), view_of(lib->P), run, ws.gsc, s, rec);
+    run_gram(view_of(ws.prep), view_of(lib->P), run, ws.gsc, s);
     if (k > 0) {
         uint32_t* idx = static_cast<uint32_t*>(ws.topk.ensure(topk_bytes(n_q, n_lib, k), "top-k"));
         float* val = reinterpret_cast<float*>(idx + (size_t)n_q * k);
-        launch_topk(scores, n_q, n_lib, k, idx, val, idx + (size_t)n_q * k * 2, s);
+        launch_topk(scores, n_q, n_lib, k, idx, val, idx + (size_t)n_q * k * 2, s,
+                    rec ? rec->clk + kClkEnd : nullptr, rec ? rec->done : nullptr);
         BS_HIP(hipGetLastError());
     }
-    if (rec) rec->mark({kBTotal1}, s);
     if (rec) {
+        rec->kind = RunRecord::kAllStages;
         rec->base.pairs = (uint64_t)n_q * n_lib;
         rec->base.main_launches = 1;
         rec->base.tile_m = 64;

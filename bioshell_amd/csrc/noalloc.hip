@@ -185,7 +185,7 @@ bs_status bs_crmsd_all_vs_all_device_noalloc(bs_context* ctx, const double* d_xy
         run.d_out = d_out_upper;
         run.out_f64 = out_f64 != 0;
         // the region's bytes held other data in earlier calls: zero it first
-        run_gram_with(v, v, run, order, n_tiles, flags, kNoAllocListCap, true, ctx->gsc.max_wg, s, nullptr);
+        run_gram_with(v, v, run, order, n_tiles, flags, kNoAllocListCap, true, ctx->gsc.max_wg, s);
     });
 }
 

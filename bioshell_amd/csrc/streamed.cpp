@@ -108,9 +108,7 @@ bs_status bs_crmsd_all_vs_all_streamed(bs_context* ctx, const double* xyz, size_
         rec->base.pairs = (uint64_t)n * (n - 1) / 2;
         rec->base.main_launches = (uint64_t)K;
         rec->base.tile_m = rec->base.tile_n = T;
-        rec->mark({kBTotal0, kBPrep0}, s);
-        prepare(ctx->prep, d, n, L, mode_of(method), nullptr, s);
-        rec->mark({kBPrep1, kBMain0}, s);
+        prepare(ctx->prep, d, n, L, mode_of(method), nullptr, s, rec->clk + kClkStart);
         auto drain = [&](int k) {  // block k's copy has been issued: wait, scatter
             BS_HIP(hipEventSynchronize(ctx->ev_copy[k % 2]));
             scatter_block(n, T, blocks[k].first, blocks[k].second,
@@ -126,8 +124,10 @@ bs_status bs_crmsd_all_vs_all_streamed(bs_context* ctx, const double* xyz, size_
             run.out_f64 = false;
             run.out_ld = T;
             run.h_count = ctx->h_blk_counts + k;
-            run_gram(view_of(ctx->prep, bi * T, T), view_of(ctx->prep, bj * T, T), run, ctx->gsc, s,
-                     nullptr);
+            if (k == 0 || k == K - 1) run.clk = rec->clk;
+            run.clk_main = k == 0;
+            run.clk_resolve = run.ends_call = k == K - 1;
+            run_gram(view_of(ctx->prep, bi * T, T), view_of(ctx->prep, bj * T, T), run, ctx->gsc, s);
             BS_HIP(hipEventRecord(ctx->ev_compute[slot], s));
             if (k >= 2) drain(k - 2);  // pinned slot free
             const int nr = std::min(T, n - bi * T);
@@ -136,13 +136,12 @@ bs_status bs_crmsd_all_vs_all_streamed(bs_context* ctx, const double* xyz, size_
             BS_HIP(hipMemcpyAsync(ctx->h_blk[slot], dev[slot], bytes, hipMemcpyDeviceToHost, cs));
             BS_HIP(hipEventRecord(ctx->ev_copy[slot], cs));
         }
-        rec->mark({kBMain1, kBFallback0, kBFallback1, kBTotal1}, s);
+        rec->kind = RunRecord::kTwoStages;
         for (int k = std::max(0, K - 2); k < K; ++k) drain(k);
         BS_HIP(hipStreamSynchronize(s));
         uint64_t flagged = 0;
         for (int k = 0; k < K; ++k) flagged += ctx->h_blk_counts[k];
         rec->base.flagged_pairs = flagged;
-        rec->gram = false;  // flagged_pairs is final in base
     });
 }
 

@@ -77,8 +77,9 @@ typedef struct bs_library bs_library;
 typedef struct bs_server bs_server;
 
 /* Timings and counters of the last all-vs-all / batch / query call on a
- * context.  Times are device times from HIP events on the context's stream
- * (adjacent stage boundaries share one event; a batch times only its total). */
+ * context.  Times are device times that the call's own kernels take from the
+ * device's wall clock (10 ns), each stage from the start of its first kernel to
+ * the start of the next stage's (a batch times only its total). */
 typedef struct bs_run_stats {
     double total_ms;        /* first prep kernel start .. last kernel end      */
     double prep_ms;         /* centring, reference fit, packing, flag clear    */
