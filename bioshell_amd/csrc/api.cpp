@@ -124,7 +124,7 @@ bs_status bs_context_create(int device, size_t hbm_budget_bytes, bs_context** ou
         ctx->ws_out.bind(&ctx->budget);
         ctx->ws_misc.bind(&ctx->budget);
         ctx->ws_stats.bind(&ctx->budget);
-        ctx->ws_clock.bind(&ctx->budget);
+        ctx->ws_clock.bind(&ctx->uncapped);
         ctx->batch.bind(&ctx->budget);
         *out = ctx.release();
     });

@@ -319,7 +319,22 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
     RunRecord* rec = ctx->begin_record();
     rec->base.pairs = n >= 2 ? (uint64_t)n * (n - 1) / 2 : 0;
     if (n >= 2 && !is_gram(m)) {
-        launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s, rec->clk, rec->done);
+        bool exact = m == BS_FP64_PLAIN;
+        if (exact) {
+            try {
+                (void)ctx->prep.cent.ensure(exact_scratch_bytes(n, L, ctx->n_cu), "centroids");
+            } catch (const Error& e) {
+                // an HBM budget without room for the centroids leaves FP64 to
+                // the per-pair kernel, which needs no workspace
+                if (e.code != BS_ERR_OUT_OF_BUDGET) throw;
+                exact = false;
+            }
+        }
+        if (exact)
+            launch_exact_avsa(d_xyz, n, L, d_out, out_f64, ctx->n_cu, ctx->prep.cent.as<double>(), s, rec->clk,
+                              rec->done);
+        else
+            launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s, rec->clk, rec->done);
         BS_HIP(hipGetLastError());
         rec->kind = RunRecord::kOneStage;
         rec->base.main_launches = 1;

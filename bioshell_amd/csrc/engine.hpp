@@ -245,6 +245,7 @@ struct bs_context {
     // clocks: kClkWords per record, those of the batch graphs (which write to
     // the clock of their replay, not of a record), the calls' zero word
     bs::DevBuf ws_clock;
+    bs::Budget uncapped{0};            // ws_clock's 8 KiB: a capped context times its calls too
     uint64_t batch_replays = 0;        // batch graphs launched, as the device counts them
     uint64_t* batch_clocks() { return ws_clock.as<uint64_t>() + kRing * bs::kClkWords; }
     static constexpr size_t kRing = 64;

@@ -22,6 +22,13 @@ namespace bs {
 // zero word.
 void launch_plain_avsa(const double* xyz, int n, int L, bool fp64, void* out, bool out_f64,
                        int n_cu, hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
+// FP64 over one ensemble with the covariance on the matrix unit
+// (kernels_exact.hip); scratch holds exact_scratch_bytes (0 for the small
+// ensembles that take one launch).
+size_t exact_scratch_bytes(int n, int L, int n_cu);
+bool exact_small(int n, int L, int n_cu);
+void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
+                       hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
 int plain_block(int n, bool fp64, bool alone, int n_cu);
 inline int plain_tiles_per_side(int n, int r) { return (n + 16 * r - 1) / (16 * r); }
 // One ensemble of a batched plain launch (f32 output); nt tiles per side.

@@ -135,17 +135,11 @@ bs_status bs_crmsd_all_vs_all_device_noalloc(bs_context* ctx, const double* d_xy
         DeviceGuard dg(ctx->device);
         const hipStream_t s = ctx->stream;
         const int n = (int)n_conf, L = (int)n_atoms;
-        if (!is_gram(method)) {  // the per-pair kernel needs no workspace
-            launch_plain_avsa(d_xyz, n, L, method == BS_FP64_PLAIN, d_out_upper, out_f64 != 0, ctx->n_cu, s);
+        if (method == BS_FP32_PLAIN) {  // needs no workspace
+            launch_plain_avsa(d_xyz, n, L, false, d_out_upper, out_f64 != 0, ctx->n_cu, s);
             BS_HIP(hipGetLastError());
             return;
         }
-        const size_t need = noalloc_scratch_bytes(n_conf, n_atoms);
-        if (need > kScratchBytes)
-            fail(BS_ERR_OUT_OF_BUDGET,
-                 "%zu x %zu needs %zu bytes of workspace; the no-allocation entry point has %zu "
-                 "(bs_crmsd_all_vs_all_device allocates what it needs)",
-                 n_conf, n_atoms, need, kScratchBytes);
         char* base = nullptr;
         {
             std::lock_guard<std::mutex> g(g_mu);
@@ -155,6 +149,18 @@ bs_status bs_crmsd_all_vs_all_device_noalloc(bs_context* ctx, const double* d_xy
                      hipGetErrorString(ctx->device >= 0 && ctx->device < kMaxDevices ? g_status[ctx->device]
                                                                                      : hipErrorInvalidDevice));
         }
+        if (method == BS_FP64_PLAIN) {  // at most 32 bytes for each of 2^21 conformations
+            static_assert(kScratchBytes >= (size_t)32 << 21, "room for the centroids");
+            launch_exact_avsa(d_xyz, n, L, d_out_upper, out_f64 != 0, ctx->n_cu, reinterpret_cast<double*>(base), s);
+            BS_HIP(hipGetLastError());
+            return;
+        }
+        const size_t need = noalloc_scratch_bytes(n_conf, n_atoms);
+        if (need > kScratchBytes)
+            fail(BS_ERR_OUT_OF_BUDGET,
+                 "%zu x %zu needs %zu bytes of workspace; the no-allocation entry point has %zu "
+                 "(bs_crmsd_all_vs_all_device allocates what it needs)",
+                 n_conf, n_atoms, need, kScratchBytes);
         // carve the regions in a fixed order, each 256-byte aligned
         const PreparedSizes z = prepared_sizes(n, L);
         const int tiles = (n + kTileRows - 1) / kTileRows;

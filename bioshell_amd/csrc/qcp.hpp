@@ -155,6 +155,16 @@ BS_HD void key_matrix(const T* M, T K[4][4])
     K[3][0] = xy - yx;      K[3][1] = zx + xz;       K[3][2] = yz + zy;       K[3][3] = -xx - yy + zz;
 }
 
+// The largest eigenvalue of the key matrix by Jacobi.
+template <class T>
+BS_HD T qcp_polish(const T* M)
+{
+    T K[4][4], q[4], lam;
+    key_matrix(M, K);
+    top_eigvec4(K, q, &lam);
+    return lam;
+}
+
 // Textbook QCP; returns RMSD.  M row-major (M[3p+q] = sum a_p b_q) of centred
 // sets, Ga, Gb their inner products, n the atom count.
 template <class T>
@@ -191,12 +201,7 @@ BS_HD T qcp_rmsd(const T* M, T Ga, T Gb, int n, int max_iter = 50)
     const T scale = fabs(T(4) * l * l * l) + fabs(T(2) * c2 * l) + fabs(c1);
     bool polish = it > 8 || fabs(dp) <= T(1e-4) * scale;
     if constexpr (sizeof(T) == 4) polish = polish || (E0 - l) < T(1e-3) * E0;
-    if (polish) {
-        T K[4][4], q[4], lam;
-        key_matrix(M, K);
-        top_eigvec4(K, q, &lam);
-        l = lam;
-    }
+    if (polish) l = qcp_polish(M);
     T r2 = T(2) * (E0 - l) / T(n);
     return sqrt(r2 > T(0) ? r2 : T(0));
 }

@@ -59,8 +59,8 @@ typedef int32_t bs_status;
 #define BS_ERR_IO (-10)   /* a file could not be read or written */
 
 /* How the pairwise cRMSD is evaluated.
- *  BS_FP64_PLAIN   per-pair kernel, FP64: centre, 3x3 covariance, QCP, sqrt.
- *  BS_FP32_PLAIN   the same kernel in FP32.
+ *  BS_FP64_PLAIN   every pair in FP64: centre, 3x3 covariance, QCP, sqrt.
+ *  BS_FP32_PLAIN   the same in FP32, by a per-pair kernel.
  *  BS_FP32_GRAM    covariance as a Gram contraction on FP32 MFMA, FP64 QCP epilogue.
  *  BS_BF16X3_GRAM  covariance as a Gram contraction on BF16 MFMA with hi/lo
  *                  split operands (hi*hi + hi*lo + lo*hi, FP32 accumulation),

@@ -357,3 +357,52 @@ def test_streamed_plain_and_errors(gpu_ctx):
         B.crmsd_all_vs_all_streamed(x, tile=100, ctx=gpu_ctx)  # not a multiple of 64
     with pytest.raises(B.BioshellGpuError):
         B.crmsd_all_vs_all_streamed(x, tile=0, ctx=gpu_ctx)
+
+
+@pytest.mark.parametrize("n,L", [(2, 1), (2, 2), (3, 3), (2, 76), (15, 4), (16, 5), (17, 7), (33, 8), (31, 9), (50, 16),
+                                 (64, 211), (33, 212), (65, 213), (2, 2600), (351, 40), (355, 17), (513, 76), (360, 97),
+                                 (505, 33)])
+def test_fp64_shapes(gpu_ctx, n, L):
+    """FP64 at the edges of its kernels (16- and 32-conformation tiles, chunks
+    of 8 and groups of 4 atoms, the one-launch form's atom count and its last
+    full round) against the oracle.  The largest eigenvalue carries a rounding
+    error of some thousand ulp at worst (the polynomial is trusted down to
+    P' = 1e-4 of its terms), so RMSD^2 one of 1e4 eps (G_a + G_b) / L."""
+    import torch
+
+    x = B.generate_ensemble(n * 31 + L, n, L, sigma=(0.5, 3.0))
+    want = O.all_vs_all(x, nthreads=8)
+    got = B.crmsd_all_vs_all(x, B.Method.FP64_PLAIN, out_f64=True, ctx=gpu_ctx).upper
+    g = ((x - x.mean(1, keepdims=True)) ** 2).sum((1, 2)).max()
+    d = 1e4 * np.finfo(np.float64).eps * 2 * g / L
+    tol = np.minimum(np.sqrt(d), d / np.maximum(want, 1e-300)) + 1e-12
+    assert (np.abs(got - want) <= tol).all()
+    # f32 output, and the entry point that allocates nothing: the same values
+    f32 = B.crmsd_all_vs_all(x, B.Method.FP64_PLAIN, ctx=gpu_ctx).upper
+    assert np.array_equal(f32, got.astype(np.float32))
+    dx = torch.from_numpy(x).cuda()
+    out = torch.zeros(len(want), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    from bioshell_amd import _native
+    import ctypes
+    B.check(_native.lib().bs_crmsd_all_vs_all_device_noalloc(
+        gpu_ctx.handle, ctypes.c_void_p(dx.data_ptr()), n, L, 0, ctypes.c_void_p(out.data_ptr()), 1))
+    gpu_ctx.synchronize()
+    assert np.array_equal(out.cpu().numpy(), got)
+
+
+def test_fp64_without_budget():
+    """FP64 on device buffers ran without any workspace: a context whose budget
+    has no room for the centroids still runs it."""
+    import torch
+
+    n, L = 600, 50
+    x = B.generate_ensemble(3, n, L, sigma=(0.5, 3.0))
+    dx = torch.from_numpy(x).cuda()
+    out = torch.zeros(n * (n - 1) // 2, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    with B.Context(0, hbm_budget_bytes=64) as ctx:
+        B.crmsd_all_vs_all_device(dx.data_ptr(), n, L, out.data_ptr(), B.Method.FP64_PLAIN, out_f64=True, ctx=ctx)
+        ctx.synchronize()
+        assert ctx.bytes_in_use() == 0
+    assert np.abs(out.cpu().numpy() - O.all_vs_all(x, nthreads=8)).max() <= 1e-5
