@@ -205,6 +205,9 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     BS_REQUIRE(!stats || (run.triangle && !run.out_f64 && run.st_min && run.st_max),
                "row statistics need the f32 triangle");
     g.stats_part = run.stats_part;
+    g.quads = !run.triangle && A.n <= 32 ? 2 : 4;
+    g.n_full = stats && run.stats_banks < 2 ? n_tiles : gram_full_tiles(n_tiles, g.quads, g.max_wg / 2);
+    g.stats_banks = g.n_full < n_tiles ? 2 : 1;
     g.stats_T = (A.n + kTileRows - 1) / kTileRows;
     g.t_start = run.clk && run.clk_main ? run.clk + kClkMain : nullptr;
 
@@ -212,7 +215,7 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     BS_HIP(hipGetLastError());
     // the statistics of the pairs the epilogue kept, as keys; the resolve
     // kernel then adds the re-evaluated pairs, and the keys become f32
-    if (stats) launch_row_stats_combine(run.stats_part, A.n, run.st_min, run.st_max, s);
+    if (stats) launch_row_stats_combine(run.stats_part, g.stats_banks, A.n, run.st_min, run.st_max, s);
     launch_flag_resolve(A.xyz, A.cent, B.xyz, B.cent, A.L, ctl, list, list_cap, bits, (int64_t)n_out,
                         g.triangle, A.n, run.out_ld, run.d_out, g.out_f64, run.h_count, run.st_min,
                         run.st_max, run.clk_resolve ? run.clk : nullptr, run.ends_call && !stats, s);
@@ -347,8 +350,20 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
         run.clk = rec->clk;
         run.done = rec->done;
         if (fused) {
-            run.stats_part = static_cast<unsigned*>(
-                ctx->ws_stats.ensure(fused_stats_tiles(n) * 256 * 4, "row statistics tiles"));
+            // a second bank of tile results allows 32 x 32 tiles; an HBM
+            // budget without room for it keeps the launch at 64 x 64 ones
+            const int tiles = (int)fused_stats_tiles(n);
+            run.stats_banks = gram_full_tiles(tiles, 4, ctx->gsc.max_wg / 2) < tiles ? 2 : 1;
+            auto reserve = [&](int banks) {
+                return ctx->ws_stats.ensure((size_t)tiles * banks * 1024, "row statistics tiles");
+            };
+            try {
+                run.stats_part = static_cast<unsigned*>(reserve(run.stats_banks));
+            } catch (const Error& e) {
+                if (e.code != BS_ERR_OUT_OF_BUDGET || run.stats_banks == 1) throw;
+                run.stats_banks = 1;
+                run.stats_part = static_cast<unsigned*>(reserve(1));
+            }
             run.st_min = reinterpret_cast<unsigned*>(d_rmin);
             run.st_max = reinterpret_cast<unsigned*>(d_rmax);
         }

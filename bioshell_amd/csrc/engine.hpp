@@ -111,9 +111,10 @@ struct GramRun {
     bool out_f64 = false;
     int64_t out_ld = 0;
     // row statistics from the epilogue (triangle, f32 output): tile results
-    // (fused_stats_tiles(n) x 1 KiB) and the n keys of each statistic, which
-    // the run leaves decoded to f32
+    // (fused_stats_tiles(n) x stats_banks KiB) and the n keys of each
+    // statistic, which the run leaves decoded to f32
     unsigned* stats_part = nullptr;
+    int stats_banks = 1;
     unsigned* st_min = nullptr;
     unsigned* st_max = nullptr;
 };

@@ -16,6 +16,44 @@ constexpr int epilogue_lds_bytes()
 // LDS bytes of the epilogue's row-statistics keys (64 x 64 tile, rows padded to 65).
 constexpr int kStatsKeysBytes = 64 * 65 * 4;
 
+// P pairs of one column, solved together (their rows' residual Grams E and
+// constants c, the column's constants cj): the secular step from 0, a second
+// one where a bracket is wide, and whether each pair has to be re-evaluated in
+// FP64: no verified root, near-duplicate residuals, estimated error above tau
+// (compared squared: no FP64 sqrt), or residuals too large for the split.
+template <int P>
+__device__ __forceinline__ void solve_pairs(const double (&E)[P][9], const double (&c)[P][kNumConsts],
+                                            const double (&cj)[kNumConsts], const EpilogueLimits& lim,
+                                            PairSolve (&o)[P], bool (&flag)[P])
+{
+    SecularSystem y[P];
+    SecularBracket br[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) y[p] = secular_system(E[p], c[p], cj);
+    bool again = false;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        br[p] = secular_step(y[p], 0.0);
+        o[p] = secular_out(br[p], lim.solve_tol2L);
+        again |= !o[p].converged & br[p].pd;
+    }
+    if (again) {  // rare for a few hundred atoms; taken by waves that need it
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            if (!o[p].converged & br[p].pd) {
+                br[p] = secular_step(y[p], br[p].lo);
+                o[p] = secular_out(br[p], lim.solve_tol2L);
+            }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const double sgg = c[p][10] * cj[10];
+        const double err = lim.acc_coef * sgg;
+        flag[p] = !o[p].converged || (o[p].H < lim.dup_coef * sgg) || (err * err > lim.tau2L * o[p].rmsd2_L) ||
+                  (c[p][9] + cj[9] > lim.rep_h_max);
+    }
+}
+
 // The FP64 QCP epilogue of a TILE x TILE tile whose accumulators the calling
 // waves hold: TILE 64 is four waves of a work-group (wave w owns rows
 // 32 (w/2) .. +31 and columns 32 (w%2) .. +31), TILE 32 is one wave on its own.
@@ -82,53 +120,28 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
     for (int r = 0; r < 16; r += P) {
         const int il = il0 + 8 * (r / 4) + (r % 4);  // P = 2: r % 4 is 0 or 2, row il + 1 holds pair r + 1
         const int i = tr * TILE + il;
-        double c[P][kNumConsts];
-        SecularSystem y[P];
-        SecularBracket br[P];
+        double c[P][kNumConsts], E[P][9];
         PairSolve o[P];
+        bool flag[P];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
 #pragma unroll
             for (int q = 0; q < kNumConsts; ++q) c[p][q] = sconst[(il + p) * 12 + q];
         }
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            double E[9];
+        for (int p = 0; p < P; ++p)
 #pragma unroll
-            for (int q = 0; q < 9; ++q) E[q] = (double)acc[q][r + p];
-            y[p] = secular_system(E, c[p], cj);
-        }
-        bool again = false;
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            br[p] = secular_step(y[p], 0.0);
-            o[p] = secular_out(br[p], lim.solve_tol2L);
-            again |= !o[p].converged & br[p].pd;
-        }
-        if (again) {  // rare for a few hundred atoms; taken by waves that need it
-#pragma unroll
-            for (int p = 0; p < P; ++p)
-                if (!o[p].converged & br[p].pd) {
-                    br[p] = secular_step(y[p], br[p].lo);
-                    o[p] = secular_out(br[p], lim.solve_tol2L);
-                }
-        }
+            for (int q = 0; q < 9; ++q) E[p][q] = (double)acc[q][r + p];
+        solve_pairs<P>(E, c, cj, lim, o, flag);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const bool ok = jok && i + p < a.n_rows && (!a.triangle || i + p < j);
-            const double sgg = c[p][10] * cj[10];
-            const double err = lim.acc_coef * sgg;
-            // flag: no verified root, near-duplicate residuals, estimated
-            // error above tau (compared squared: no FP64 sqrt), or residuals
-            // too large for the split
-            const bool flag = !o[p].converged || (o[p].H < lim.dup_coef * sgg) ||
-                              (err * err > lim.tau2L * o[p].rmsd2_L) || (c[p][9] + cj[9] > lim.rep_h_max);
             const int64_t oi =
                 a.triangle ? tri_index(a.n_rows, i + p, j) : (int64_t)(i + p) * a.out_ld + j;
             if constexpr (STATS) {  // f32 output
                 const float v = __builtin_amdgcn_sqrtf((float)(o[p].rmsd2_L * lim.inv_L));
                 if (ok) static_cast<float*>(a.out)[oi] = v;
-                skeys[(il + p) * 65 + jl] = ok && !flag && v == v ? fkey(__float_as_uint(v)) : 0xFFFFFFFFu;
+                skeys[(il + p) * 65 + jl] = ok && !flag[p] && v == v ? fkey(__float_as_uint(v)) : 0xFFFFFFFFu;
             } else if (ok) {
                 if (a.out_f64)
                     static_cast<double*>(a.out)[oi] = sqrt(o[p].rmsd2_L * lim.inv_L);
@@ -136,7 +149,7 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
                     static_cast<float*>(a.out)[oi] =
                         __builtin_amdgcn_sqrtf((float)(o[p].rmsd2_L * lim.inv_L));
             }
-            flagged |= (uint32_t)(ok & flag) << (r + p);
+            flagged |= (uint32_t)(ok & flag[p]) << (r + p);
         }
     }
     // flagged pairs are rare: one branch per tile rather than a queueing
@@ -172,11 +185,15 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
         }
         if (q == 0) {
             const int64_t b = (int64_t)tr * a.stats_T - (int64_t)tr * (tr - 1) / 2 + (tc - tr);
-            unsigned* out = a.stats_part + b * 256;
+            unsigned* out = a.stats_part + b * (256 * a.stats_banks);
             out[r] = lo;
             out[64 + r] = hi;
             out[128 + r] = clo;
             out[192 + r] = chi;
+            if (a.stats_banks == 2) {
+                out[256 + r] = out[384 + r] = 0xFFFFFFFFu;
+                out[320 + r] = out[448 + r] = 0u;
+            }
         }
     }
 }

@@ -121,6 +121,8 @@ struct GramArgs {
     int n_kblk;             // atom blocks of 16
     const uint32_t* tiles;  // (tile_row << 16 | tile_col) per logical tile
     int n_tiles;
+    int n_full;             // the first n_full as 64 x 64 tiles, the rest as 32 x 32 tiles,
+    int quads;              // `quads` each: 4, or the upper 2 where there are at most 32 rows
     int triangle;           // 1: packed upper triangle of rows==cols, only i<j
     int64_t out_ld;         // dense output: row stride (triangle: ignored)
     void* out;
@@ -137,10 +139,13 @@ struct GramArgs {
     int max_wg;             // resident work-groups (2 per CU)
     // Row statistics from the epilogue (triangle, f32 output): when set, tile
     // (tr, tc) writes the 256 keys of row_stats_tile_kernel's layout to
-    // stats_part + 256 (tr stats_T - tr (tr - 1) / 2 + tc - tr), leaving out
-    // the flagged pairs (the resolve kernel adds their final values).
+    // stats_part + 256 stats_banks (tr stats_T - tr (tr - 1) / 2 + tc - tr),
+    // leaving out the flagged pairs (the resolve kernel adds their final
+    // values).  With two banks the right half's row keys and the lower half's
+    // column keys of a tile split into 32 x 32 ones go to the second.
     unsigned* stats_part;
     int stats_T;            // tiles per side of the triangle
+    int stats_banks;        // key banks per tile: 2 where a launch has 32 x 32 tiles, else 1
     uint64_t* t_start;      // clock word of the launch's start, or null
 };
 
@@ -148,6 +153,9 @@ struct GramArgs {
 // Returns the number of tiles written to `out` (capacity must be enough).
 int build_tile_order(int tiles_r, int tiles_c, bool triangle, int super, uint32_t* out);
 
+// How many of n_tiles tiles a launch on n_cu compute units runs as 64 x 64
+// ones (GramArgs::n_full).
+int gram_full_tiles(int n_tiles, int quads, int n_cu);
 void launch_gram(const GramArgs& a, GramMode mode, hipStream_t s);
 void launch_zero_u32(uint32_t* p, int n, hipStream_t s);
 
@@ -270,7 +278,7 @@ inline size_t fused_stats_tiles(int n)
 }
 // Combines the epilogue's tile results into keys (kmin / kmax, n each, n >= 2),
 // which the resolve kernel then updates; decode turns the keys into f32.
-void launch_row_stats_combine(const unsigned* part, int n, unsigned* kmin, unsigned* kmax, hipStream_t s);
+void launch_row_stats_combine(const unsigned* part, int banks, int n, unsigned* kmin, unsigned* kmax, hipStream_t s);
 void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end,
                              unsigned* done);
 // For each of m members, the largest distance to the other members.

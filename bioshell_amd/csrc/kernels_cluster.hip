@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void row_stats_tile_kernel(const float* __rest
 // in LDS with the element's keys so far: the keys of f32::MAX and -f32::MAX
 // for the first chunk, else the values rmin / rmax hold.  The last chunk
 // decodes the keys to f32.
-__global__ __launch_bounds__(512) void row_stats_reduce_kernel(const unsigned* __restrict__ part, int n, int T,
+__global__ __launch_bounds__(512) void row_stats_reduce_kernel(const unsigned* __restrict__ part, int banks, int n, int T,
                                                                int t0, int t1, int base, int first, int last,
                                                                unsigned* __restrict__ rmin,
                                                                unsigned* __restrict__ rmax)
@@ -132,15 +132,19 @@ __global__ __launch_bounds__(512) void row_stats_reduce_kernel(const unsigned* _
         if (t < t1) {
             const int f = tile_row_first(t, T) - base;
             for (int tc = t + q; tc < T; tc += 8) {
-                const unsigned* p = part + (size_t)(f + tc - t) * 256;
-                lo = min(lo, p[r]);
-                hi = max(hi, p[64 + r]);
+                for (int k = 0; k < banks; ++k) {
+                    const unsigned* p = part + ((size_t)(f + tc - t) * banks + k) * 256;
+                    lo = min(lo, p[r]);
+                    hi = max(hi, p[64 + r]);
+                }
             }
         }
         for (int tr = t0 + q; tr < t1 && tr <= t; tr += 8) {
-            const unsigned* p = part + (size_t)(tile_row_first(tr, T) - base + t - tr) * 256;
-            lo = min(lo, p[128 + r]);
-            hi = max(hi, p[192 + r]);
+            for (int k = 0; k < banks; ++k) {
+                const unsigned* p = part + ((size_t)(tile_row_first(tr, T) - base + t - tr) * banks + k) * 256;
+                lo = min(lo, p[128 + r]);
+                hi = max(hi, p[192 + r]);
+            }
         }
     }
     slo[q][r] = lo;
@@ -501,7 +505,7 @@ void launch_row_stats(const float* up, int n, float* rmin, float* rmax, void* sc
     auto* a = reinterpret_cast<unsigned*>(rmin);
     auto* b = reinterpret_cast<unsigned*>(rmax);
     if (n < 2) {
-        row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, n, T, 0, 0, 0, 1, 1, a, b);
+        row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, 1, n, T, 0, 0, 0, 1, 1, a, b);
         return;
     }
     // chunks of whole tile rows, each within the chunk size (or one tile row)
@@ -513,15 +517,15 @@ void launch_row_stats(const float* up, int n, float* rmin, float* rmax, void* sc
         while (t1 < T && (t1 + 1) * T - (t1 + 1) * t1 / 2 - base <= chunk) ++t1;
         const int tiles = t1 * T - t1 * (t1 - 1) / 2 - base;
         row_stats_tile_kernel<<<tiles, 256, 0, s>>>(up, n, T, base, part);
-        row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, n, T, t0, t1, base, t0 == 0, t1 == T, a, b);
+        row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, 1, n, T, t0, t1, base, t0 == 0, t1 == T, a, b);
         t0 = t1;
     }
 }
 
-void launch_row_stats_combine(const unsigned* part, int n, unsigned* kmin, unsigned* kmax, hipStream_t s)
+void launch_row_stats_combine(const unsigned* part, int banks, int n, unsigned* kmin, unsigned* kmax, hipStream_t s)
 {
     const int T = (n + 63) / 64;
-    row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, n, T, 0, T, 0, 1, 0, kmin, kmax);
+    row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, banks, n, T, 0, T, 0, 1, 0, kmin, kmax);
 }
 
 void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end, unsigned* done)

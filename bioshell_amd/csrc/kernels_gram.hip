@@ -16,32 +16,40 @@
 // through LDS.  Work-group ids are dealt to the 8 XCDs round-robin, so the
 // logical tile is taken from a contiguous per-XCD slice of a super-blocked
 // order: each XCD's L2 keeps re-using the same row and column panels.
-#include "gram_tile.hpp"
+#include "gram_split.hpp"
 
 #include <algorithm>
 
 namespace bs {
 namespace {
 
-
-
-// One work-group per 64 x 64 tile.  Work-group ids are dealt to the 8 XCDs
+// One work-group per 64 x 64 tile, then one per 32 x 32 tile of the tiles past
+// a.n_full (gram_full_tiles).  Work-group ids are dealt to the 8 XCDs
 // round-robin, so the logical tile comes from a contiguous per-XCD slice of
-// the super-blocked order.  Two work-groups share each CU; the ones in the
-// second resident batch (ids [n_cu, 2 n_cu)) start about half a tile late, so
-// that on every SIMD one work-group's MFMA phase overlaps the other's FP64
-// epilogue (VALU).  Tiles cost the same, so refilled slots keep the offset.
+// the super-blocked order.  Two work-groups share each CU, and on a SIMD one's
+// MFMA phase overlaps the other's FP64 epilogue (VALU).
 template <int MODE, bool STATS>
 __global__ __launch_bounds__(256, 2) void gram_kernel(GramArgs a)
 {
     __shared__ uint4 lds[3][4][kPanelBlockU4];  // 3 stages x (A0, A1, B0, B1) x 6 KiB
     stamp_start(a.t_start);
     const int wg = blockIdx.x;
-    const int per = (a.n_tiles + kXcd - 1) / kXcd;
-    const int t = (wg % kXcd) * per + (wg / kXcd);
-    if (t >= a.n_tiles) return;
-    const uint32_t code = a.tiles[t];
-    gram_tile64<MODE, true, 2, STATS>(a, (int)(code >> 16), (int)(code & 0xFFFFu), lds, (int)threadIdx.x);
+    const int per = (a.n_full + kXcd - 1) / kXcd;
+    if (wg < per * kXcd) {
+        const int t = (wg % kXcd) * per + (wg / kXcd);
+        if (t >= a.n_full) return;
+        const uint32_t code = a.tiles[t];
+        gram_tile64<MODE, true, 2, STATS>(a, (int)(code >> 16), (int)(code & 0xFFFFu), lds, (int)threadIdx.x);
+        return;
+    }
+    const int w = wg - per * kXcd, n_quad = a.quads * (a.n_tiles - a.n_full);
+    const int per_q = (n_quad + kXcd - 1) / kXcd;
+    const int q = (w % kXcd) * per_q + (w / kXcd);
+    if (q >= n_quad) return;
+    const uint32_t code = a.tiles[a.n_full + q / a.quads];
+    const int part = q % a.quads;
+    const int tr = 2 * (int)(code >> 16) + (part >> 1), tc = 2 * (int)(code & 0xFFFFu) + (part & 1);
+    gram_split32<MODE, STATS>(a, tr, tc, reinterpret_cast<char*>(lds), (w / kXcd) >> 5, (int)threadIdx.x);
 }
 
 __global__ void zero_u32_kernel(uint32_t* p, int n)
@@ -220,11 +228,29 @@ int build_tile_order(int tiles_r, int tiles_c, bool triangle, int super, uint32_
     return n;
 }
 
+// A 64 x 64 tile takes a CU about as long alone (bf16x3, 150 atoms: 14.5 us
+// past the launch) as two take it together (21), so a launch's last, partly
+// filled round of n_cu tiles costs as much as a full one.  As 32 x 32 tiles
+// over the idle CUs it takes 6 us with one each and 12 with two, but four
+// cost more than the tile they replace.  Measured on 256 CUs against 64 x 64
+// tiles only (bf16x3, 100 and 260 atoms): less than one round, remainders up
+// to 0.21 n_cu 1.8-2.1x faster, 0.26-0.47 1.4-1.5x, 0.53 +-3 %, 0.8 and up
+// 15-18 % slower; after one or two full rounds, up to 0.22 16-23 %, 0.27-0.48
+// 2-8 % faster, 0.6 8-13 % slower; after three or more, 0.05-0.22 8-15 % faster, 0.36 1-2 %
+// slower.  FP32: 2.4x, 1.5x; 1.16-1.46x, 1.07-1.11x; 1.03-1.16x.  From 16
+// rounds on the remainder is noise.
+int gram_full_tiles(int n_tiles, int quads, int n_cu)
+{
+    const int rem = n_tiles % n_cu, rounds = n_tiles / n_cu;
+    const int most = rounds < 3 ? 2 * n_cu : n_cu;  // 32 x 32 tiles, one or two per CU
+    return rounds < 16 && quads * rem <= most ? n_tiles - rem : n_tiles;
+}
+
 void launch_gram(const GramArgs& a, GramMode mode, hipStream_t s)
 {
     if (a.n_tiles <= 0) return;
-    const int per = (a.n_tiles + kXcd - 1) / kXcd;
-    const int grid = per * kXcd;
+    const int n_quad = a.quads * (a.n_tiles - a.n_full);
+    const int grid = ((a.n_full + kXcd - 1) / kXcd + (n_quad + kXcd - 1) / kXcd) * kXcd;
     const bool st = a.stats_part != nullptr;
     if (mode == kGramBF16x3 && st)
         gram_kernel<kGramBF16x3, true><<<grid, 256, 0, s>>>(a);

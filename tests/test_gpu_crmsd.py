@@ -359,6 +359,40 @@ def test_streamed_plain_and_errors(gpu_ctx):
         B.crmsd_all_vs_all_streamed(x, tile=0, ctx=gpu_ctx)
 
 
+@pytest.mark.parametrize("n,L", [(2, 100), (32, 17), (33, 96), (64, 81), (65, 16), (97, 113), (959, 80), (961, 85),
+                                 (1409, 100), (1437, 97), (1473, 90), (2017, 83)])
+def test_gram_tile_shapes(gpu_ctx, n, L):
+    """Where a launch changes from 64 x 64 to 32 x 32 tiles (none, all, the last
+    round; halves and quarters outside the matrix, 1 to many atom blocks)
+    against the oracle, with the row statistics of what was written."""
+    import torch
+
+    x = B.generate_ensemble(n + L, n, L, sigma=(0.5, 3.0), near_fraction=0.05)
+    want = O.all_vs_all(x, nthreads=8)
+    for method in (B.Method.FP32_GRAM, B.Method.BF16X3_GRAM):
+        assert np.abs(run(gpu_ctx, x, method) - want).max() <= TOL[method]
+    assert np.abs(run(gpu_ctx, x, B.Method.BF16X3_GRAM, out_f64=True) - want).max() <= 1e-4
+    dx = torch.from_numpy(x).cuda()
+    out, (lo, hi) = torch.zeros(len(want), device="cuda"), torch.zeros(2, n, device="cuda").unbind(0)
+    torch.cuda.synchronize()
+    B.crmsd_all_vs_all_row_stats_device(dx.data_ptr(), n, L, out.data_ptr(), lo.data_ptr(), hi.data_ptr(),
+                                        ctx=gpu_ctx)
+    gpu_ctx.synchronize()
+    full = np.zeros((n, n), np.float32)
+    full[np.triu_indices(n, 1)] = out.cpu().numpy()
+    full = full + full.T
+    assert np.array_equal(hi.cpu().numpy(), full.max(1))
+    np.fill_diagonal(full, np.inf)
+    assert np.array_equal(lo.cpu().numpy(), full.min(1))
+    # the same rows against a library: at most 32 of them, and more
+    lib = B.Library(x, ctx=gpu_ctx)
+    square = np.zeros((n, n))
+    square[np.triu_indices(n, 1)] = want
+    square = square + square.T
+    for q in (1, 32, 33):
+        assert np.abs(lib.query_all(x[:q]) - square[:q]).max() <= TOL[B.Method.BF16X3_GRAM]
+
+
 @pytest.mark.parametrize("n,L", [(2, 1), (2, 2), (3, 3), (2, 76), (15, 4), (16, 5), (17, 7), (33, 8), (31, 9), (50, 16),
                                  (64, 211), (33, 212), (65, 213), (2, 2600), (351, 40), (355, 17), (513, 76), (360, 97),
                                  (505, 33)])
