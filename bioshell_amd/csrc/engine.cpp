@@ -173,8 +173,8 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     // kernel then re-evaluates them in FP64 and leaves the region clean.
     const uint64_t n_out =
         run.triangle ? (uint64_t)A.n * (A.n - 1) / 2 : (uint64_t)A.n * (uint64_t)run.out_ld;
-    uint32_t* ctl = flags;  // count, report, done, spare
-    int64_t* list = reinterpret_cast<int64_t*>(flags + 4);
+    uint32_t* ctl = flags;
+    int64_t* list = reinterpret_cast<int64_t*>(flags + kFlagCtlWords);
     uint32_t* bits = reinterpret_cast<uint32_t*>(list + list_cap);
     if (clear_flags) launch_zero_words(flags, (int64_t)(flag_region_bytes(n_out, list_cap) / 4), s);
 
@@ -197,8 +197,8 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     g.out_f64 = run.out_f64 ? 1 : 0;
     g.flag_bits = bits;
     g.flag_list = list;
-    g.flag_count = ctl;
-    g.flag_cap = list_cap;
+    g.flag_ctl = ctl;
+    g.flag_cap = list_cap / kFlagLists;
     g.lim = epilogue_limits(gram_thresholds(A.mode, A.L, A.n_kblk), A.L);
     g.max_wg = max_wg > 0 ? max_wg : 512;
     const bool stats = run.stats_part != nullptr;
@@ -216,7 +216,7 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
     // the statistics of the pairs the epilogue kept, as keys; the resolve
     // kernel then adds the re-evaluated pairs, and the keys become f32
     if (stats) launch_row_stats_combine(run.stats_part, g.stats_banks, A.n, run.st_min, run.st_max, s);
-    launch_flag_resolve(A.xyz, A.cent, B.xyz, B.cent, A.L, ctl, list, list_cap, bits, (int64_t)n_out,
+    launch_flag_resolve(A.xyz, A.cent, B.xyz, B.cent, A.L, ctl, list, g.flag_cap, bits, (int64_t)n_out,
                         g.triangle, A.n, run.out_ld, run.d_out, g.out_f64, run.h_count, run.st_min,
                         run.st_max, run.clk_resolve ? run.clk : nullptr, run.ends_call && !stats, s);
     if (stats)

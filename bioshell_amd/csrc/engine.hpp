@@ -174,13 +174,13 @@ struct RunRecord {
 // rows of A x cols of B (or the upper triangle of A when triangle).  Asynchronous.
 // Words of the flag bitmap of n_out outputs (a whole number of 16-byte units).
 inline uint64_t flag_words(uint64_t n_out) { return ((n_out + 31) / 32 + 3) / 4 * 4; }
-// Bytes of the flag region: four control words (count, report, done, spare),
-// list_cap queued entries, then the bitmap.  The list sits at a fixed offset
+// Bytes of the flag region: the control words, list_cap queued entries (a
+// multiple of kFlagLists), then the bitmap.  The list sits at a fixed offset
 // and the bitmap grows at the end, so a region reused for a larger launch
 // never finds list entries where its bitmap is.
 inline size_t flag_region_bytes(uint64_t n_out, int list_cap)
 {
-    return 16 + (size_t)list_cap * 8 + (size_t)flag_words(n_out) * 4;
+    return (size_t)kFlagCtlWords * 4 + (size_t)list_cap * 8 + (size_t)flag_words(n_out) * 4;
 }
 // The Gram launch sequence with every buffer given: `order` (n_tiles tile
 // codes on the device), `flags` (flag_region_bytes(n_out, list_cap)); no

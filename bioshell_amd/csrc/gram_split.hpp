@@ -200,14 +200,10 @@ __device__ __forceinline__ void gram_split32(const GramArgs& a, int tr, int tc, 
             flagged |= (uint32_t)(ok & flag[p]) << (k + p);
         }
     }
-    if (flagged) {
-#pragma unroll 1
-        for (int k = 0; k < 4; ++k) {
-            if (!((flagged >> k) & 1u)) continue;
-            const int i = tr * 32 + (t >> 5) + 8 * k;
-            flag_output(a, true, a.triangle ? tri_index(a.n_rows, i, j) : (int64_t)i * a.out_ld + j);
-        }
-    }
+    flag_pairs<4>(a, flagged, lane, [&](int k) {
+        const int i = tr * 32 + (t >> 5) + 8 * k;
+        return a.triangle ? tri_index(a.n_rows, i, j) : (int64_t)i * a.out_ld + j;
+    });
     if constexpr (STATS) {
         __syncthreads();
         // tile row r and tile column r: eight threads of four entries each

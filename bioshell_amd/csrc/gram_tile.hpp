@@ -154,14 +154,10 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
     }
     // flagged pairs are rare: one branch per tile rather than a queueing
     // branch per pair (those cost about a sixth of the epilogue)
-    if (flagged) {
-#pragma unroll 1
-        for (int r = 0; r < 16; ++r) {
-            if (!((flagged >> r) & 1u)) continue;
-            const int i = tr * TILE + il0 + 8 * (r / 4) + (r % 4);
-            flag_output(a, true, a.triangle ? tri_index(a.n_rows, i, j) : (int64_t)i * a.out_ld + j);
-        }
-    }
+    flag_pairs<16>(a, flagged, lane, [&](int r) {
+        const int i = tr * TILE + il0 + 8 * (r / 4) + (r % 4);
+        return a.triangle ? tri_index(a.n_rows, i, j) : (int64_t)i * a.out_ld + j;
+    });
     if constexpr (STATS) {
         __syncthreads();  // every wave's keys are in LDS
         // tile row r and tile column r: four threads of 16 entries each, then two shuffles

@@ -128,11 +128,11 @@ struct GramArgs {
     void* out;
     int out_f64;
     uint32_t* flag_bits;    // bit o set: output o is re-evaluated in FP64
-    // when flag_list is set, flagged outputs are queued there first
-    // (*flag_count counts every flagged output; the bitmap takes those
-    // beyond flag_cap)
+    // when flag_list is set, flagged outputs are queued there first: kFlagLists
+    // lists of flag_cap entries with their control words at flag_ctl (the
+    // bitmap takes those beyond a list's capacity)
     int64_t* flag_list;
-    uint32_t* flag_count;
+    uint32_t* flag_ctl;
     int flag_cap;
     EpilogueLimits lim;     // flagging limits and the RMSD scale
     // launch shape
@@ -160,11 +160,11 @@ void launch_gram(const GramArgs& a, GramMode mode, hipStream_t s);
 void launch_zero_u32(uint32_t* p, int n, hipStream_t s);
 
 // FP64 re-evaluation of the outputs the Gram kernel flagged, from raw
-// coordinates and centroids of rows (a) and columns (b): one wave per entry of
-// `list` (min(count, cap) entries), then, only when count > cap, a scan of the
-// bitmap `bits` (n_out bits) that clears every word it reads.  ctl holds
-// count, report, done: the last work-group to finish copies count to report
-// and zeroes count and done, so the region is ready for the next launch.  It
+// coordinates and centroids of rows (a) and columns (b): the entries of the
+// kFlagLists lists at `list` (`cap` entries each), then, only when a list
+// overflowed, the set bits of the bitmap `bits` (n_out bits), which it clears.
+// The last work-group to finish leaves the total count in the control words
+// `ctl` and zeroes the others, so the region is ready for the next launch.  It
 // also stores the count into h_report when given (a pinned host word, written
 // with a system-scope store: no separate device-to-host copy).  clk (a call's
 // clock, or null) gets the launch's start and end, the count and, with
@@ -181,7 +181,15 @@ void launch_flag_resolve(const double* xyz_a, const double* cent_a, const double
 // into list (cap entries), clearing the queued ones; *count += set bits.
 void launch_flag_compact(uint32_t* bits, int64_t n_words, int64_t* list, int cap, uint32_t* count,
                          hipStream_t s);
-constexpr int kFlagListCap = 1 << 20;  // queued FP64 re-evaluations per call (8 MiB)
+constexpr int kFlagListCap = (1 << 20) - 128;  // queued FP64 re-evaluations per call (8 MiB with the control words)
+// A Gram launch's queue is kFlagLists lists of equal capacity, work-group b
+// appending to list b % kFlagLists: atomics on one word follow each other 9 ns
+// apart, which for 2112 waves was 18 us of a launch of 2000 x 20 atoms (48 us,
+// 30 without them).  Control words of list k, from 16 k on (a cache line of
+// their own): entries counted, work-groups of the re-evaluation done; of list
+// 0 also: lists done, entries counted in all (the report).
+constexpr int kFlagLists = 16;
+constexpr int kFlagCtlWords = 16 * kFlagLists;
 void launch_zero_words(uint32_t* p, int64_t n_words, hipStream_t s);
 
 // Per-query top-k over a dense n_q x n_lib score matrix (ascending, ties by index).

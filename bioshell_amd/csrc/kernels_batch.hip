@@ -173,59 +173,41 @@ __global__ __launch_bounds__(256, 2) void batch_gram_kernel(BatchArgs b)
 }
 
 // ------------------------------------------------------------------ FP64 re-evaluation
-// Flagged pair of ensemble E at output o: one wave, FP64 textbook QCP.
-__device__ inline void batch_eval_one(const BatchEns& E, int64_t o, int lane)
+// The lane's flagged pair (a batch-wide bit index, or -1).
+__device__ inline void batch_eval(const BatchArgs& b, int64_t gb, int lane)
 {
-    const int i = tri_row(o, E.n);
-    const int j = (int)(o - ((int64_t)i * E.n - (int64_t)i * (i + 1) / 2)) + i + 1;
-    const double r = fallback_pair(E.xyz + (int64_t)i * E.L * 3, E.cent + 3 * (int64_t)i,
-                                   E.xyz + (int64_t)j * E.L * 3, E.cent + 3 * (int64_t)j, E.L,
-                                   lane);
-    if (lane == 0) E.out[o] = (float)r;
-}
-
-// The queued entries (batch-wide bit indices), one wave each.
-__global__ __launch_bounds__(256) void batch_flag_eval_kernel(BatchArgs b)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t m = min((int64_t)b.counters[kXcd], (int64_t)kFlagListCap);
-    for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < m; k += (int64_t)gridDim.x * 4) {
-        const int64_t gb = b.flag_list[k];
+    PairRef p{nullptr, nullptr, nullptr, nullptr, 0};
+    float* out = nullptr;
+    if (gb >= 0) {
         const int64_t gw = gb >> 5;
         const int e = find_ens(b.word_prefix, b.n_ens, gw);
         const BatchEns& E = b.ens[e];
         const int64_t o = (gw - b.word_prefix[e]) * 32 + (gb & 31);
-        if (o < (int64_t)E.n * (E.n - 1) / 2) batch_eval_one(E, o, lane);
-    }
-}
-
-// Bits the queue could not hold: each wave takes 64 consecutive words of the
-// batch-wide bitmap (one per lane) and re-evaluates their set bits one pair
-// at a time.
-__global__ __launch_bounds__(256) void batch_fallback_kernel(BatchArgs b)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t n_waves = (int64_t)gridDim.x * 4;
-    const uint32_t* bits0 = b.ens_bits0;
-    for (int64_t w0 = wave * 64; w0 < b.total_words; w0 += n_waves * 64) {
-        const int64_t wi = w0 + lane;
-        uint32_t word = wi < b.total_words ? bits0[wi] : 0u;
-        while (true) {
-            const uint64_t m = __ballot(word != 0u);
-            if (!m) break;
-            const int src = __ffsll((unsigned long long)m) - 1;
-            const uint32_t wsrc = __shfl(word, src);
-            const int bit = __ffs(wsrc) - 1;
-            if (lane == src) word &= word - 1u;  // clear the lowest set bit
-            const int64_t gw = w0 + src;
-            const int e = find_ens(b.word_prefix, b.n_ens, gw);
-            const BatchEns& E = b.ens[e];
-            const int64_t o = (gw - b.word_prefix[e]) * 32 + bit;
-            if (o >= (int64_t)E.n * (E.n - 1) / 2) continue;
-            batch_eval_one(E, o, lane);
+        if (o < (int64_t)E.n * (E.n - 1) / 2) {
+            const int i = tri_row(o, E.n);
+            const int j = (int)(o - ((int64_t)i * E.n - (int64_t)i * (i + 1) / 2)) + i + 1;
+            p = {E.xyz + (int64_t)i * E.L * 3, E.xyz + (int64_t)j * E.L * 3, E.cent + 3 * (int64_t)i,
+                 E.cent + 3 * (int64_t)j, E.L};
+            out = E.out + o;
         }
     }
+    const double r = fallback_pairs(p, lane);
+    if (out) *out = (float)r;
+}
+
+// The queued entries (batch-wide bit indices), then, only when there were more
+// than the queue holds, the bitmap's remaining bits: each wave takes 64
+// consecutive words of the batch-wide bitmap at a time.
+__global__ __launch_bounds__(256) void batch_resolve_kernel(BatchArgs b)
+{
+    __shared__ uint16_t slots[4][2048];
+    const int lane = threadIdx.x & 63;
+    const int wave = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), n_waves = (int)gridDim.x * 4;
+    const uint32_t cnt = b.counters[kXcd];
+    FlagCursor cur(b.flag_list, min(cnt, (uint32_t)kFlagListCap), wave, n_waves,
+                   cnt > (uint32_t)kFlagListCap ? b.ens_bits0 : nullptr, b.total_words, wave, n_waves,
+                   slots[threadIdx.x >> 6], lane);
+    for (int64_t gb; cur.next(gb);) batch_eval(b, gb, lane);
 }
 
 // The graph's last node: the start word, the time this kernel starts and the
@@ -270,10 +252,7 @@ void launch_batch_gram(const BatchArgs& b, uint32_t* zero_base, int64_t zero_wor
 void launch_batch_fallback(const BatchArgs& b, hipStream_t s)
 {
     launch_flag_compact(b.ens_bits0, b.total_words, b.flag_list, kFlagListCap, b.counters + kXcd, s);
-    batch_flag_eval_kernel<<<1024, 256, 0, s>>>(b);
-    const int64_t waves = (b.total_words + 63) / 64;
-    const int64_t blocks = std::min<int64_t>(2048, std::max<int64_t>(1, (waves + 3) / 4));
-    batch_fallback_kernel<<<(int)blocks, 256, 0, s>>>(b);
+    batch_resolve_kernel<<<512, 256, 0, s>>>(b);
     batch_report_kernel<<<1, 1, 0, s>>>(b);
 }
 

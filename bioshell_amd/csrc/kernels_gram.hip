@@ -121,94 +121,74 @@ __device__ inline void decode_output(int64_t o, int triangle, int n, int64_t out
     }
 }
 
-// FP64 re-evaluation of one flagged output o (lane 0 stores the result and,
-// with st_min set, folds the stored f32 value into both elements' keys).
-__device__ inline void resolve_output(int64_t o, const double* __restrict__ xa, const double* __restrict__ ca,
-                                      const double* __restrict__ xb, const double* __restrict__ cb, int L,
-                                      int triangle, int n, int64_t out_ld, void* __restrict__ out, int out_f64,
-                                      unsigned* st_min, unsigned* st_max, int lane)
-{
-    int i, j;
-    decode_output(o, triangle, n, out_ld, i, j);
-    const double r = fallback_pair(xa + (int64_t)i * L * 3, ca + 3 * (int64_t)i, xb + (int64_t)j * L * 3,
-                                   cb + 3 * (int64_t)j, L, lane);
-    if (lane == 0) {
-        if (out_f64) {
-            static_cast<double*>(out)[o] = r;
-        } else {
-            const float v = (float)r;
-            static_cast<float*>(out)[o] = v;
-            if (st_min && v == v) {
-                const unsigned k = fkey(__float_as_uint(v));
-                atomicMin(st_min + i, k);
-                atomicMin(st_min + j, k);
-                atomicMax(st_max + i, k);
-                atomicMax(st_max + j, k);
-            }
-        }
-    }
-}
+// The flagged outputs of one Gram launch, up to 64 per wave at a time: the
+// queued entries, work-group b taking its part of list b % kFlagLists, then,
+// only when a list overflowed, a scan of the bitmap in which each wave takes 64
+// words and clears them.  The last work-group to finish publishes the count
+// and zeroes the other control words for the next launch; the groups count
+// themselves done per list, then the lists (on one word their atomics, 9 ns
+// apart, made an empty list take 3.7 us; this way 2.2).
+constexpr int kResolveWaves = 4;  // per work-group
 
-// The flagged outputs of one Gram launch: one wave per queued entry, then,
-// only when more were flagged than the list holds, a scan of the bitmap in
-// which each wave takes 64 words (one per lane), processes their set bits one
-// pair at a time (the 64 lanes splitting the atoms) and clears the words.
-// ctl = {count, report, done}: the last work-group to finish publishes the
-// count in report and zeroes count and done for the next launch.
-__global__ __launch_bounds__(256) void flag_resolve_kernel(const double* __restrict__ xa,
-                                                           const double* __restrict__ ca,
-                                                           const double* __restrict__ xb,
-                                                           const double* __restrict__ cb, int L,
-                                                           uint32_t* __restrict__ ctl,
-                                                           const int64_t* __restrict__ list, int cap,
-                                                           uint32_t* __restrict__ bits, int64_t n_out,
-                                                           int triangle, int n, int64_t out_ld,
-                                                           void* __restrict__ out, int out_f64,
-                                                           uint32_t* h_report, unsigned* st_min,
-                                                           unsigned* st_max, uint64_t* clk, int ends_call)
+__global__ __launch_bounds__(64 * kResolveWaves) void flag_resolve_kernel(
+    const double* __restrict__ xa, const double* __restrict__ ca, const double* __restrict__ xb,
+    const double* __restrict__ cb, int L, uint32_t* __restrict__ ctl, const int64_t* __restrict__ list, int cap,
+    uint32_t* __restrict__ bits, int64_t n_out, int triangle, int n, int64_t out_ld, void* __restrict__ out,
+    int out_f64, uint32_t* h_report, unsigned* st_min, unsigned* st_max, uint64_t* clk, int ends_call)
 {
+    __shared__ uint16_t slots[kResolveWaves][2048];
     stamp_start(clk ? clk + kClkResolve : nullptr);
     const int lane = threadIdx.x & 63;
-    const uint32_t cnt = ctl[0];  // read before this group counts itself done
-    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t n_waves = (int64_t)gridDim.x * 4;
-    const int64_t m = min((int64_t)cnt, (int64_t)cap);
-    for (int64_t k = wave; k < m; k += n_waves) {
-        const int64_t o = list[k];
-        if (o >= 0 && o < n_out)
-            resolve_output(o, xa, ca, xb, cb, L, triangle, n, out_ld, out, out_f64, st_min, st_max, lane);
-    }
-    if ((int64_t)cnt > (int64_t)cap) {  // uniform: the bitmap holds the rest
-        const int64_t n_words = (n_out + 31) >> 5;
-        for (int64_t w0 = wave * 64; w0 < n_words; w0 += n_waves * 64) {
-            const int64_t wi = w0 + lane;
-            uint32_t word = wi < n_words ? bits[wi] : 0u;
-            if (word) bits[wi] = 0u;
-            while (true) {
-                const uint64_t msk = __ballot(word != 0u);
-                if (!msk) break;
-                const int src = __ffsll((unsigned long long)msk) - 1;
-                const uint32_t wsrc = __shfl(word, src);
-                const int bit = __ffs(wsrc) - 1;
-                const int64_t o = (w0 + src) * 32 + bit;
-                if (lane == src) word &= word - 1u;  // clear the lowest set bit
-                if (o >= n_out) continue;
-                resolve_output(o, xa, ca, xb, cb, L, triangle, n, out_ld, out, out_f64, st_min, st_max, lane);
-            }
+    const int seg = (int)blockIdx.x % kFlagLists, w = threadIdx.x >> 6;
+    // read before this group counts itself done
+    const uint32_t mine = lane < kFlagLists ? ctl[16 * lane] : 0u;
+    const bool overflow = __any(mine > (uint32_t)cap);
+    const uint32_t cnt = __builtin_amdgcn_readlane(mine, seg);
+    FlagCursor cur(list + (int64_t)seg * cap, min(cnt, (uint32_t)cap), (int)blockIdx.x / kFlagLists * kResolveWaves + w,
+                   (int)gridDim.x / kFlagLists * kResolveWaves, overflow ? bits : nullptr, (n_out + 31) >> 5,
+                   (int)blockIdx.x * kResolveWaves + w, (int)gridDim.x * kResolveWaves, slots[w], lane);
+    for (int64_t o; __builtin_expect(cur.next(o), 0);) {
+        PairRef p{xa, xb, ca, cb, 0};
+        int i = 0, j = 0;
+        if (o >= 0 && o < n_out) {
+            decode_output(o, triangle, n, out_ld, i, j);
+            p = {xa + (int64_t)i * L * 3, xb + (int64_t)j * L * 3, ca + 3 * (int64_t)i, cb + 3 * (int64_t)j, L};
+        }
+        const double r = fallback_pairs(p, lane);
+        if (!p.L) continue;
+        if (out_f64) {
+            static_cast<double*>(out)[o] = r;
+            continue;
+        }
+        const float v = (float)r;
+        static_cast<float*>(out)[o] = v;
+        // the stored value joins both elements' keys, which only fall (rise):
+        // one already beyond it needs no atomic
+        if (st_min && v == v) {
+            const unsigned k = fkey(__float_as_uint(v));
+            if (k < st_min[i]) atomicMin(st_min + i, k);
+            if (k < st_min[j]) atomicMin(st_min + j, k);
+            if (k > st_max[i]) atomicMax(st_max + i, k);
+            if (k > st_max[j]) atomicMax(st_max + j, k);
         }
     }
-    // Every thread of the group has used its copy of the count (no fence:
+    // Every thread of the group has used its copy of the counts (no fence:
     // the reset only needs the reads done, and the next launch sees it).
     __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(&ctl[2], 1u) == gridDim.x - 1) {
-        ctl[1] = cnt;
-        ctl[0] = 0u;
+    if (threadIdx.x >= 64) return;
+    uint32_t all = mine;
+#pragma unroll
+    for (int d = 1; d < kFlagLists; d <<= 1) all += (uint32_t)__shfl_xor((int)all, d);
+    if (threadIdx.x == 0 && atomicAdd(&ctl[16 * seg + 1], 1u) == gridDim.x / kFlagLists - 1 &&
+        atomicAdd(&ctl[2], 1u) == kFlagLists - 1) {
         ctl[2] = 0u;
-        if (h_report) __hip_atomic_store(h_report, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        ctl[3] = all;
+        for (int k = 0; k < kFlagLists; ++k) ctl[16 * k] = ctl[16 * k + 1] = 0u;
+        if (h_report) __hip_atomic_store(h_report, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (clk) {
             const uint64_t now = wall_clock64();
             clk[kClkResolveEnd] = now;
-            clk[kClkCount] = cnt;
+            clk[kClkCount] = all;
             if (ends_call) clk[kClkEnd] = now;
         }
     }
@@ -281,11 +261,14 @@ void launch_flag_resolve(const double* xyz_a, const double* cent_a, const double
                          int out_f64, uint32_t* h_report, unsigned* st_min, unsigned* st_max,
                          uint64_t* clk, bool ends_call, hipStream_t s)
 {
-    // 1024 waves: a typical list (tens to thousands of pairs) is one pass, a
-    // full list or a bitmap scan takes several.  A grid sized for the bitmap
-    // (up to 1024 groups) cost 9 us more per call in dispatch and in the
-    // done-counter atomics of the idle groups.
-    flag_resolve_kernel<<<256, 256, 0, s>>>(
+    // 1024 waves: a typical list (tens to thousands of pairs) is one trip of a
+    // few pairs per wave.  Short chains flag up to half of their pairs and
+    // get twice as many where there is enough to do (2000 x 20 370 -> 299 us,
+    // 6000 x 60 84 -> 58; four times as many: 264 and 55, but 22 instead of 15
+    // for 2000 x 60).
+    const int groups = L <= kShortChain && n_out >= (int64_t)1 << 19 ? 512 : 256;
+    static_assert(256 % kFlagLists == 0, "every list has the same number of groups");
+    flag_resolve_kernel<<<groups, 64 * kResolveWaves, 0, s>>>(
         xyz_a, cent_a, xyz_b, cent_b, L, ctl, list, cap, bits, n_out, triangle, n, out_ld, out, out_f64,
         h_report, st_min, st_max, clk, ends_call ? 1 : 0);
 }

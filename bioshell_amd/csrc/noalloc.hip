@@ -26,7 +26,7 @@ namespace bs {
 namespace {
 
 constexpr size_t kScratchBytes = size_t(64) << 20;  // 64 MiB per GPU
-constexpr int kNoAllocListCap = 1 << 16;           // queued FP64 re-evaluations (512 KiB); more go
+constexpr int kNoAllocListCap = (1 << 16) - 128;   // queued FP64 re-evaluations (512 KiB); more go
                                                    // through the bitmap scan
 constexpr int kMaxDevices = 64;
 constexpr int kTileRows = 64;

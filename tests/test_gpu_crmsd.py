@@ -359,6 +359,38 @@ def test_streamed_plain_and_errors(gpu_ctx):
         B.crmsd_all_vs_all_streamed(x, tile=0, ctx=gpu_ctx)
 
 
+@pytest.mark.parametrize("n,L", [(2, 5), (33, 12), (700, 8), (700, 31), (700, 33), (300, 63), (300, 64), (300, 65),
+                                 (130, 150)])
+def test_flagged_pairs_by_length(gpu_ctx, n, L):
+    """Rigid copies of two chains, all pairs flagged: at the lengths where the
+    re-evaluation changes its split over the lanes, in numbers that fill the
+    smaller queue of the entry point without allocations (n 700), against the
+    oracle, and the same values from that entry point, a batch of mixed
+    lengths and the blocks of a streamed call."""
+    import ctypes
+
+    import torch
+    from bioshell_amd import _native
+
+    x = np.concatenate([B.generate_ensemble(L, n // 2, L, sigma=0.0), B.generate_ensemble(L + 1, n - n // 2, L, sigma=0.0)])
+    want = O.all_vs_all(x, nthreads=8)
+    got = B.crmsd_all_vs_all(x, ctx=gpu_ctx).upper
+    assert gpu_ctx.last_stats()["flagged_pairs"] >= (n // 2) * (n // 2 - 1) // 2
+    assert np.abs(got - want).max() <= TOL[B.Method.BF16X3_GRAM]
+    dx, out = torch.from_numpy(x).cuda(), torch.zeros(len(want), device="cuda")
+    torch.cuda.synchronize()
+    B.check(_native.lib().bs_crmsd_all_vs_all_device_noalloc(
+        gpu_ctx.handle, ctypes.c_void_p(dx.data_ptr()), n, L, int(B.Method.BF16X3_GRAM),
+        ctypes.c_void_p(out.data_ptr()), 0))
+    gpu_ctx.synchronize()
+    assert np.array_equal(out.cpu().numpy(), got)
+    other = B.generate_ensemble(3, 40, 90, sigma=0.0)
+    batch = B.crmsd_batch([other, x, other[:, :20]], ctx=gpu_ctx)
+    assert np.array_equal(batch[1], got)
+    assert np.abs(batch[0] - O.all_vs_all(other)).max() <= TOL[B.Method.BF16X3_GRAM]
+    assert np.array_equal(B.crmsd_all_vs_all_streamed(x, tile=64, ctx=gpu_ctx).upper, got)
+
+
 @pytest.mark.parametrize("n,L", [(2, 100), (32, 17), (33, 96), (64, 81), (65, 16), (97, 113), (959, 80), (961, 85),
                                  (1409, 100), (1437, 97), (1473, 90), (2017, 83)])
 def test_gram_tile_shapes(gpu_ctx, n, L):
