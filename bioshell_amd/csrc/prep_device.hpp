@@ -24,6 +24,8 @@
 // runs once per ensemble, none of it per pair.
 #pragma once
 
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "qcp.hpp"
 #include "wave.hpp"
@@ -238,6 +240,72 @@ __device__ inline void fit_reduce(const double (&v)[NV], Lds& lds, int c, int g)
     __syncthreads();
 }
 
+// A thread's conformation: the work-group's first one (uniform) and the byte
+// offset from it, so that a load's address is one 32-bit register.
+struct FitSource {
+    const char* base;
+    unsigned off;
+    bool live;
+};
+
+// Atoms k, k + 16, ... (N of them) of conformation x, zeros for those at or
+// past L and for a conformation that is not live.  Every call issues the same
+// loads (addresses clamped to atom 0), so that the wait for one register set
+// never has to drain the loads of another. 
+template <int N>
+__device__ __forceinline__ void load_atoms(const FitSource& x, int k, int L, double (&d)[N][3])
+{
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const bool in = x.live & (k + kFitLanes * u < L);
+        const double* p =
+            reinterpret_cast<const double*>(x.base + (x.off + (in ? 24u * (unsigned)(k + kFitLanes * u) : 0u)));
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const double v = p[q];
+            d[u][q] = in ? v : 0.0;
+        }
+    }
+}
+
+// A first pass over a thread's atoms: atom(x_k, y_k) for its atoms k = g,
+// g + 16, ... in order, y a set shared by the conformations (at yb).
+// The plain loop leaves the atoms past a multiple of eight to a loop of one
+// load, one wait each: up to seven, and all seven where only some threads have
+// an eighth.  There (four or more) the last atoms are taken eight or four at a
+// time too, those past L as zeros: 120 atoms, 500 conformations: 33 -> 26 us
+// for all four launches.  For fewer the plain loop is as good or better (150
+// and 300 atoms: 0.6 and 1.7 us of 32 and 62).
+template <class F>
+__device__ __forceinline__ void fit_first_pass(const FitSource& x, const double* __restrict__ yb, int L, int g, F atom)
+{
+    const int blocks = (L + kFitLanes - 1) / kFitLanes, tail = blocks % 8;
+    if (tail == 0 ? L % kFitLanes == 0 : tail < 4) {
+        if (!x.live) return;
+        const double* xp = reinterpret_cast<const double*>(x.base + x.off);
+#pragma unroll 8
+        for (int k = g; k < L; k += kFitLanes) {
+            const double b[3] = {xp[3 * k], xp[3 * k + 1], xp[3 * k + 2]};
+            const double a[3] = {yb[3 * k], yb[3 * k + 1], yb[3 * k + 2]};
+            atom(b, a);
+        }
+        return;
+    }
+    const FitSource y{reinterpret_cast<const char*>(yb), 0u, x.live};
+    auto step = [&](auto count, int k) {
+        constexpr int N = decltype(count)::value;
+        double b[N][3], a[N][3];
+        load_atoms(x, k, L, b);
+        load_atoms(y, k, L, a);
+#pragma unroll
+        for (int u = 0; u < N; ++u) atom(b[u], a[u]);
+    };
+    int k = 0;
+#pragma unroll 1
+    for (; blocks * kFitLanes - k > 4 * kFitLanes; k += 8 * kFitLanes) step(std::integral_constant<int, 8>{}, k + g);
+    if (k < blocks * kFitLanes) step(std::integral_constant<int, 4>{}, k + g);
+}
+
 // Reference mean, stage 1 -- slice s of an ensemble of n conformations:
 // samples 16 s .. 16 s + 15 (those below S).  For each sample, the centroid
 // c and, from the covariance of the centred sets,
@@ -252,45 +320,31 @@ __device__ inline void fit0_slice(const double* __restrict__ xyz, int n, int S, 
     const int tid = threadIdx.x, c = tid / kFitLanes, g = tid % kFitLanes;
     const int t0 = s * kFitConfs;
     const bool live = t0 + c < S;
-    const double* x = xyz + (int64_t)(live ? ref_sample_index(t0 + c, n, S) : 0) * L * 3;
+    // (a slice's 16 samples lie within 16 (n / S + 1) conformations, n / S < 9)
+    const int first = ref_sample_index(t0, n, S);
+    const FitSource x{reinterpret_cast<const char*>(xyz + (int64_t)first * L * 3),
+                      live ? 24u * (unsigned)(ref_sample_index(t0 + c, n, S) - first) * (unsigned)L : 0u, live};
     {
         double v[17];
 #pragma unroll
         for (int q = 0; q < 17; ++q) v[q] = 0.0;
-        if (live) {
-#pragma unroll 8
-            for (int k = g; k < L; k += kFitLanes) {
-                const double b0 = x[3 * k], b1 = x[3 * k + 1], b2 = x[3 * k + 2];
-                const double a0 = xyz[3 * k], a1 = xyz[3 * k + 1], a2 = xyz[3 * k + 2];
-                v[0] += b0; v[1] += b1; v[2] += b2;
-                v[3] += a0; v[4] += a1; v[5] += a2;
-                v[6] += b0 * a0; v[7] += b0 * a1; v[8] += b0 * a2;
-                v[9] += b1 * a0; v[10] += b1 * a1; v[11] += b1 * a2;
-                v[12] += b2 * a0; v[13] += b2 * a1; v[14] += b2 * a2;
-                v[15] += b0 * b0 + b1 * b1 + b2 * b2;
-                v[16] += a0 * a0 + a1 * a1 + a2 * a2;
+        fit_first_pass(x, xyz, L, g, [&](const double (&b)[3], const double (&a)[3]) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                v[p] += b[p];
+                v[3 + p] += a[p];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) v[6 + 3 * p + q] += b[p] * a[q];
             }
-        }
+            v[15] += b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
+            v[16] += a[0] * a[0] + a[1] * a[1] + a[2] * a[2];
+        });
         fit_reduce(v, lds, c, g);
     }
     // the second pass's chunks: kPer atoms per thread
     constexpr int kPer = kFitMeanAtoms / kFitLanes;
     double xc[kPer][3], xn[kPer][3];
-    // every call issues the same 3 kPer loads (addresses clamped to atom 0,
-    // values zeroed): the wait for one register set never drains the other's
-    auto load = [&](int k0, double (&dst)[kPer][3]) {
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int k = k0 + g + kFitLanes * u;
-            const bool in = live && k < L;
-            const int kk = in ? k : 0;
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const double v = x[3 * kk + q];
-                dst[u][q] = in ? v : 0.0;
-            }
-        }
-    };
+    auto load = [&](int k0, double (&dst)[kPer][3]) { load_atoms(x, k0 + g, L, dst); };
     load(0, xc);  // in flight while the rotations are solved
     __builtin_amdgcn_sched_barrier(0);
     if (tid < kFitConfs) {
@@ -471,43 +525,29 @@ __device__ inline void fit_pack_block(const double* __restrict__ xyz, const doub
     const int tid = threadIdx.x, c = tid / kFitLanes, g = tid % kFitLanes;
     const int i = i0 + c;
     const bool live = i < n;
-    const double* x = xyz + (int64_t)(live ? i : 0) * L * 3;
+    const FitSource x{reinterpret_cast<const char*>(xyz + (int64_t)min(i0, n - 1) * L * 3),
+                      live ? 24u * (unsigned)c * (unsigned)L : 0u, live};
+    const FitSource r{reinterpret_cast<const char*>(ref), 0u, live};
     {
         double v[13];
 #pragma unroll
         for (int q = 0; q < 13; ++q) v[q] = 0.0;
-        if (live) {
-#pragma unroll 8
-            for (int k = g; k < L; k += kFitLanes) {
-                const double b0 = x[3 * k], b1 = x[3 * k + 1], b2 = x[3 * k + 2];
-                const double a0 = ref[3 * k], a1 = ref[3 * k + 1], a2 = ref[3 * k + 2];
-                v[0] += b0; v[1] += b1; v[2] += b2;
-                v[3] += b0 * a0; v[4] += b0 * a1; v[5] += b0 * a2;
-                v[6] += b1 * a0; v[7] += b1 * a1; v[8] += b1 * a2;
-                v[9] += b2 * a0; v[10] += b2 * a1; v[11] += b2 * a2;
-                v[12] += b0 * b0 + b1 * b1 + b2 * b2;
+        fit_first_pass(x, ref, L, g, [&](const double (&b)[3], const double (&a)[3]) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                v[p] += b[p];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) v[3 + 3 * p + q] += b[p] * a[q];
             }
-        }
+            v[12] += b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
+        });
         fit_reduce(v, lds, c, g);
     }
     // pass 2's chunks: x and r of one atom per block, kFitChunk blocks
     double xb[kFitChunk][3], rb[kFitChunk][3], xn[kFitChunk][3], rn[kFitChunk][3];
-    // Every call issues the same 6 kFitChunk loads (addresses clamped to atom
-    // 0, values zeroed), so that the wait for one register set never has to
-    // drain the loads of the other.
     auto load = [&](int kb0, double (&xd)[kFitChunk][3], double (&rd)[kFitChunk][3]) {
-#pragma unroll
-        for (int kbl = 0; kbl < kFitChunk; ++kbl) {
-            const int k = (kb0 + kbl) * kAtomBlock + g;
-            const bool in = live && kb0 + kbl < n_kblk && k < L;
-            const int kk = in ? k : 0;
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const double xv = x[3 * kk + q], rv = ref[3 * kk + q];
-                xd[kbl][q] = in ? xv : 0.0;
-                rd[kbl][q] = in ? rv : 0.0;
-            }
-        }
+        load_atoms(x, kb0 * kAtomBlock + g, L, xd);
+        load_atoms(r, kb0 * kAtomBlock + g, L, rd);
     };
     load(0, xb, rb);  // in flight while the rotations are solved
     __builtin_amdgcn_sched_barrier(0);
