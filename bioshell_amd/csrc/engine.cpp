@@ -54,14 +54,9 @@ PrepView prepare_into(const PreparedPtrs& p, const double* d_xyz, int n, int L, 
                       const double* fixed_ref, hipStream_t s, uint64_t* t_start)
 {
     const int n_pad = round_up(n, kTileRows), n_kblk = (L + kAtomBlock - 1) / kAtomBlock;
-    const double* ref = fixed_ref;  // a fixed reference is read in place
-    if (!fixed_ref) {
-        launch_reference(d_xyz, n, L, p.partial, p.ref, s, t_start);
-        t_start = nullptr;
-        ref = p.ref;
-    }
-    launch_fit_pack(d_xyz, ref, n, n_pad, L, n_kblk, mode, p.rot, p.cent, p.panels, p.consts, n_pad, s,
-                    t_start);
+    // a fixed reference is read in place
+    launch_prepare(d_xyz, n, L, n_pad, n_kblk, mode, fixed_ref, p.partial, p.ref, p.rot, p.cent, p.panels, p.consts,
+                   n_pad, s, t_start);
     BS_HIP(hipGetLastError());
     return prep_view(p, d_xyz, n, L, mode);
 }

@@ -87,16 +87,15 @@ __host__ __device__ inline int ref_sample_index(int s, int n, int S)
     return (int)((int64_t)s * n / S);
 }
 
-// Reference of one ensemble (prep_device.hpp): for the S = ref_sample_count(n)
-// samples, the slices' partial sums of the fitted samples (partial,
-// ref_slices(S) x 3L), then r (ref: 3L values) and R0 (6).
-void launch_reference(const double* xyz, int n, int L, double* partial, double* ref, hipStream_t s,
-                      uint64_t* t_start);
-// Fit onto ref and pack: rotations (rot), centroids (cent), operand panels of
-// e_i = rot_i (x_i - c_i) - ref and the constants, for n_pad rows.
-void launch_fit_pack(const double* xyz, const double* ref, int n, int n_pad, int L, int n_kblk,
-                     GramMode mode, double* rot, double* cent, void* panels, double* consts, int ld,
-                     hipStream_t s, uint64_t* t_start);
+// Preparation of one ensemble (prep_device.hpp).  The reference, unless a fixed
+// one is given: for the S = ref_sample_count(n) samples, the slices' partial
+// sums of the fitted samples (partial, ref_slices(S) x 3L), then r (ref: 3L
+// values) and R0 (6).  Then the fit onto it and the packing: rotations (rot),
+// centroids (cent), operand panels of e_i = rot_i (x_i - c_i) - ref and the
+// constants, for n_pad rows.
+void launch_prepare(const double* xyz, int n, int L, int n_pad, int n_kblk, GramMode mode, const double* fixed_ref,
+                    double* partial, double* ref, double* rot, double* cent, void* panels, double* consts, int ld,
+                    hipStream_t s, uint64_t* t_start);
 
 // The epilogue's flagging limits and RMSD scale at one atom count L, formed
 // on the host so that the kernels hold them in scalar registers rather than

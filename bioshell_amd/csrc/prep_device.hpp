@@ -439,6 +439,19 @@ __device__ inline void mean_final_coord(const double* __restrict__ partial, int 
     ref[v] = (((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]))) / S;
 }
 
+// The same for at most N slices, all loads in flight at once (a slice past the
+// last adds zero).
+template <int N>
+__device__ inline double mean_few_slices(const double* __restrict__ partial, int n_slices, int S, int L, int v)
+{
+    double x[N], acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < N; ++u) x[u] = partial[v + min(u, n_slices - 1) * 3 * (int64_t)L];
+#pragma unroll
+    for (int u = 0; u < N; ++u) acc[u & 7] += u < n_slices ? x[u] : 0.0;
+    return (((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]))) / S;
+}
+
 // Work-group ids are dealt to the 8 XCDs in turn.  A grid of 8 * per
 // work-groups maps id b to the logical block (b % 8) * per + b / 8, so that
 // each XCD packs a contiguous range of conformations: the panel words of one
@@ -517,7 +530,7 @@ __device__ inline void store_image(const uint4* img, int nkb, uint4* __restrict_
 // g = |e~|^2 and C = sum r e~^T and drops each operand value into the LDS
 // image of the chunk's panel words, which the work-group then writes out.
 template <int MODE>
-__device__ inline void fit_pack_block(const double* __restrict__ xyz, const double* __restrict__ ref,
+__device__ __forceinline__ void fit_pack_block(const double* __restrict__ xyz, const double* __restrict__ ref,
                                       int n, int L, int n_kblk, int i0, double* __restrict__ rot,
                                       double* __restrict__ cent, uint4* __restrict__ panels,
                                       double* __restrict__ consts, int ld, FitPackLds& lds)

@@ -150,6 +150,17 @@ def test_batch_device_entry(gpu_ctx, batch):
             assert np.array_equal(t.cpu().numpy(), h), f"replay {rep}"
 
 
+@pytest.mark.parametrize("n,L", [(70, 10), (70, 113), (66, 832), (66, 833), (1040, 60), (2056, 20), (2300, 20),
+                                 (4104, 8), (4240, 8)])
+def test_batch_equals_single_preparation(gpu_ctx, n, L):
+    """A single call forms the reference in its own way at most 832 atoms and 32
+    slices of samples (4111 conformations), with other loads up to 16 slices
+    (2055): the values are those of a batch, bit for bit."""
+    x = B.generate_ensemble(n + L, n, L, sigma=(0.5, 3.0))
+    single = B.crmsd_all_vs_all(x, B.Method.FP32_GRAM, ctx=gpu_ctx).upper
+    assert np.array_equal(B.crmsd_batch([x], B.Method.FP32_GRAM, ctx=gpu_ctx)[0], single)
+
+
 def test_batch_flagged_pairs_reevaluated(gpu_ctx):
     """Exact duplicates inside ensembles are flagged and re-evaluated in FP64."""
     xs = []
