@@ -32,13 +32,13 @@ template <int MODE, bool STATS>
 __global__ __launch_bounds__(256, 2) void gram_kernel(GramArgs a)
 {
     __shared__ uint4 lds[3][4][kPanelBlockU4];  // 3 stages x (A0, A1, B0, B1) x 6 KiB
-    stamp_start(a.t_start);
     const int wg = blockIdx.x;
     const int per = (a.n_full + kXcd - 1) / kXcd;
     if (wg < per * kXcd) {
         const int t = (wg % kXcd) * per + (wg / kXcd);
         if (t >= a.n_full) return;
         const uint32_t code = a.tiles[t];
+        stamp_start(a.t_start);  // after the read, which a store before it would make per lane
         gram_tile64<MODE, true, 2, STATS>(a, (int)(code >> 16), (int)(code & 0xFFFFu), lds, (int)threadIdx.x);
         return;
     }
@@ -48,6 +48,7 @@ __global__ __launch_bounds__(256, 2) void gram_kernel(GramArgs a)
     if (q >= n_quad) return;
     const uint32_t code = a.tiles[a.n_full + q / a.quads];
     const int part = q % a.quads;
+    stamp_start(a.t_start);
     const int tr = 2 * (int)(code >> 16) + (part >> 1), tc = 2 * (int)(code & 0xFFFFu) + (part & 1);
     gram_split32<MODE, STATS>(a, tr, tc, reinterpret_cast<char*>(lds), (w / kXcd) >> 5, (int)threadIdx.x);
 }
