@@ -89,6 +89,27 @@ def test_topk_selection_is_exact_over_chunks(gpu_ctx, n_base, copies, k):
     lib.close()
 
 
+@pytest.mark.parametrize("n,k,copies", [(1, 1, 1), (40, 40, 1), (257, 128, 1), (1025, 129, 1), (8192, 512, 3), (8193, 513, 1),
+                                        (16384, 1024, 1), (16385, 100, 40), (32768, 100, 4), (32768, 1, 32768),
+                                        (32768, 300, 700), (32769, 100, 700)])
+def test_topk_row_sizes(gpu_ctx, n, k, copies):
+    """The first k of a full sort by (value, index) of the same scores, at the
+    sizes where the selection changes: keys per thread, candidates, ways of
+    sorting them, more equal values than candidates, one work-group or chunks."""
+    base = B.generate_ensemble(n + k, (n + copies - 1) // copies, 70, sigma=(0.5, 3.0))
+    x = np.tile(base, (copies, 1, 1))[:n]
+    lib = B.Library(x, ctx=gpu_ctx)
+    q = B.generate_ensemble(5, 3, 70, sigma=(0.5, 3.0))
+    q[1] = x[n // 2]
+    scores = lib.query_all(q)
+    idx, val = lib.query_topk(q, k)
+    for r in range(3):
+        order = np.lexsort((np.arange(n), scores[r]))[:k]
+        assert np.array_equal(idx[r], order)
+        assert np.array_equal(val[r], scores[r][order])
+    lib.close()
+
+
 def test_topk_argument_errors(gpu_ctx, bucket):
     lib_x, q, _ = bucket
     lib = B.Library(lib_x[:50], ctx=gpu_ctx)
