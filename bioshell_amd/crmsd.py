@@ -398,8 +398,8 @@ class Library:
     def query_topk(self, q, k: int = 100) -> tuple[np.ndarray, np.ndarray]:
         """Per query, the k members of lowest cRMSD: (idx u32, rmsd f32), each (n_q, k)."""
         q = self._queries(q)
-        idx = np.empty((q.shape[0], k), dtype=np.uint32)
-        val = np.empty((q.shape[0], k), dtype=np.float32)
+        both = np.empty((2, q.shape[0], k), dtype=np.uint32)  # adjacent: one copy from the device
+        idx, val = both[0], both[1].view(np.float32)
         check(_native.lib().bs_query_topk(self.ctx.handle, self.handle, _dp(q), q.shape[0], k,
                                           idx.ctypes.data_as(_native.c_u32p), val.ctypes.data_as(_native.c_fp)))
         return idx, val

@@ -203,8 +203,10 @@ bs_status bs_query_topk(bs_context* ctx, bs_library* lib, const double* q_xyz, s
         enqueue_query(lib, ctx->qws, q_xyz, (int)n_q, (int)k, s, ctx->begin_record());
         const uint32_t* d_idx = ctx->qws.topk.as<uint32_t>();
         const float* d_val = reinterpret_cast<const float*>(d_idx + n_q * k);
-        BS_HIP(hipMemcpyAsync(idx, d_idx, n_q * k * 4, hipMemcpyDeviceToHost, s));
-        BS_HIP(hipMemcpyAsync(rmsd, d_val, n_q * k * 4, hipMemcpyDeviceToHost, s));
+        // the device's two arrays are adjacent: one copy where the caller's are too
+        const bool adjacent = reinterpret_cast<const char*>(rmsd) == reinterpret_cast<const char*>(idx) + n_q * k * 4;
+        BS_HIP(hipMemcpyAsync(idx, d_idx, n_q * k * (adjacent ? 8 : 4), hipMemcpyDeviceToHost, s));
+        if (!adjacent) BS_HIP(hipMemcpyAsync(rmsd, d_val, n_q * k * 4, hipMemcpyDeviceToHost, s));
         BS_HIP(hipStreamSynchronize(s));
     });
 }
