@@ -4,15 +4,17 @@
 // bioshell-pdb/src/calc/transformation.rs:22-37, applied as at 171-174), the
 // RMSD of the fit and, optionally, the superposed coordinates R x + t.
 //
-// The reference is centred once (one block).  Then one launch does the rest:
-// a work-group of 256 threads takes C = 256 / G conformations, G threads each
+// One launch does it: a work-group of 256 threads takes C = 256 / G
+// conformations, G threads each
 // (G = sup_lanes(L)), and every thread keeps its up to 8 atoms in registers,
 // so a conformation is read from HBM once and its superposed copy written
 // once (24 L bytes each way).  The sums (centroid, M = sum x r_c^T, |x|^2)
 // are reduced through LDS, one thread per conformation solves the rotation
 // (rotation_fast, Newton from E0 = (G_x + G_r) / 2) and the RMSD, and every
-// thread writes R x + t for its atoms.  Chains longer than 2048 atoms take
-// three passes (covariance per block, Jacobi per thread, apply per atom).
+// thread writes R x + t for its atoms.  Every wave centres the reference for
+// itself, while its conformations are on their way; above 512 atoms, where
+// that is many loads a lane, one block does so in a launch before.  Chains
+// longer than 2048 atoms take three passes (covariance per block, Jacobi per thread, apply per atom).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -166,9 +168,13 @@ __global__ __launch_bounds__(256) void sup_apply_kernel(const double* __restrict
 }
 
 // ---------------------------------------------------------------- fused form
-constexpr int kSupAtoms = 8;                 // atoms per thread held in registers
+constexpr int kSupAtoms = 8;                 // atoms per thread held in registers, at most
+// With at most this many a fourth work-group fits on a CU (10,000 x 300: 42.6 ->
+// 40.2 us); above 512 atoms it spilled and lost (1000 x 600: 13.6 -> 14.3).
+constexpr int kSupFewAtoms = 5;
 constexpr int kSupResidentMax = 256 * kSupAtoms;
-constexpr int kSupValues = 13;               // sum d (3), sum d r_c^T (9), sum |d|^2; d = x - x_0
+constexpr int kSupValues = 14;               // sum d (3), sum d r_c^T (9), sum |d|^2, sum |r_c|^2; d = x - x_0
+constexpr int kSupFoldLanes = 64;            // up to this G the waves centre the reference
 
 int sup_lanes(int L)
 {
@@ -178,20 +184,25 @@ int sup_lanes(int L)
 }
 
 struct SupLds {
-    double red[256 * kSupValues + 256];  // G (13 C + 1) partials
+    double red[256 * kSupValues + 256];  // G (14 C + 1) partials
     double part2[16 * kSupValues];
     double tot[16][kSupValues];
     double rt[16][12];  // R | t of the work-group's conformations
+    double rc[3];       // the reference's centroid
 };
 
-template <int G>
-__global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict__ xyz, int n, int L,
-                                                        const double* __restrict__ ref_c,
+// ref: the reference itself (G <= kSupFoldLanes), else its centred copy, with
+// its centroid at info.  Bound by memory: 10,000 x 300 is 144 MB (28 us at a
+// copy's rate) in 40 us, 42 with the reference centred by a launch of its own,
+// 3000 x 120 in 9 and 12.
+template <int G, int A>
+__global__ __launch_bounds__(256, A <= kSupFewAtoms ? 4 : 3) void sup_fused_kernel(const double* __restrict__ xyz, int n, int L,
+                                                        const double* __restrict__ ref,
                                                         const double* __restrict__ info,
                                                         double* __restrict__ rot, double* __restrict__ trans,
                                                         double* __restrict__ rmsd, double* __restrict__ out)
 {
-    constexpr int C = 256 / G, A = kSupAtoms, S = kSupValues * C + 1, PARTS = G / 16;
+    constexpr int C = 256 / G, S = kSupValues * C + 1, PARTS = G / 16;
     constexpr int PAIRS = kSupValues * C;
     __shared__ SupLds lds;
     const int tid = threadIdx.x, c = tid / G, g = tid % G;
@@ -207,20 +218,44 @@ __global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict
     for (int q = 0; q < kSupValues; ++q) v[q] = 0.0;
 #pragma unroll
     for (int j = 0; j < A; ++j) {
-        const int k = g + G * j;
-        xv[j][0] = xv[j][1] = xv[j][2] = 0.0;
-        if (live && k < L) {
-            xv[j][0] = x[3 * k];
-            xv[j][1] = x[3 * k + 1];
-            xv[j][2] = x[3 * k + 2];
+        if (G * j >= L) break;  // uniform
+        const double* p = x + 3 * min(g + G * j, L - 1);
+        xv[j][0] = p[0];
+        xv[j][1] = p[1];
+        xv[j][2] = p[2];
+    }
+    double rc[3] = {0.0, 0.0, 0.0};  // the reference's centroid
+    if constexpr (G <= kSupFoldLanes) {
+#pragma unroll
+        for (int j = 0; j < (G * A + 63) / 64; ++j) {
+            if (64 * j >= L) break;  // uniform
+            const int k = (tid & 63) + 64 * j;
+            const double* r = ref + 3 * min(k, L - 1);
+            const double r0 = r[0], r1 = r[1], r2 = r[2];
+            rc[0] += k < L ? r0 : 0.0;
+            rc[1] += k < L ? r1 : 0.0;
+            rc[2] += k < L ? r2 : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            rc[q] = wave_sum(rc[q]) / L;
+            if (tid == 0) lds.rc[q] = rc[q];  // for the solve, where registers are short
         }
     }
 #pragma unroll
     for (int j = 0; j < A; ++j) {
+        if (G * j >= L) break;
         const int k = g + G * j;
-        if (live && k < L) {
+        const double* r = ref + 3 * min(k, L - 1);
+        double a0 = r[0], a1 = r[1], a2 = r[2];
+        if constexpr (G <= kSupFoldLanes) {
+            a0 -= rc[0];
+            a1 -= rc[1];
+            a2 -= rc[2];
+        }
+        if (k < L) {
+            v[13] += a0 * a0 + a1 * a1 + a2 * a2;
             const double b0 = xv[j][0] - o0, b1 = xv[j][1] - o1, b2 = xv[j][2] - o2;
-            const double a0 = ref_c[3 * k], a1 = ref_c[3 * k + 1], a2 = ref_c[3 * k + 2];
             v[0] += b0; v[1] += b1; v[2] += b2;
             v[3] += b0 * a0; v[4] += b0 * a1; v[5] += b0 * a2;
             v[6] += b1 * a0; v[7] += b1 * a1; v[8] += b1 * a2;
@@ -258,6 +293,7 @@ __global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict
         double R[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1}, t[3] = {0, 0, 0};
         if (m < n) {
             const double* sm = lds.tot[tid];
+            const double* cr = G > kSupFoldLanes ? info : lds.rc;
             const double* xm = xyz + m * 3 * (int64_t)L;
             const double dc[3] = {sm[0] / L, sm[1] / L, sm[2] / L};  // c - x_0
             const double cc[3] = {xm[0] + dc[0], xm[1] + dc[1], xm[2] + dc[2]};
@@ -265,10 +301,10 @@ __global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict
 #pragma unroll
             for (int q = 0; q < 9; ++q) M[q] = sm[3 + q];  // r_c is centred: sum (x - c) r_c^T
             const double gx = sm[12] - L * (dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
-            rotation_fast(M, R, 0.5 * (gx + info[3]));
+            rotation_fast(M, R, 0.5 * (gx + sm[13]));
 #pragma unroll
             for (int r = 0; r < 3; ++r)
-                t[r] = info[r] - (R[3 * r] * cc[0] + R[3 * r + 1] * cc[1] + R[3 * r + 2] * cc[2]);
+                t[r] = cr[r] - (R[3 * r] * cc[0] + R[3 * r + 1] * cc[1] + R[3 * r + 2] * cc[2]);
             // sum r_c^T R (x - c) = sum_ab R_ab M_ba
             double lam = 0.0;
 #pragma unroll
@@ -282,7 +318,7 @@ __global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict
 #pragma unroll
                 for (int r = 0; r < 3; ++r) trans[3 * m + r] = t[r];
             if (rmsd) {
-                const double r2 = (gx + info[3] - 2.0 * lam) / L;
+                const double r2 = (gx + sm[13] - 2.0 * lam) / L;
                 rmsd[m] = sqrt(r2 > 0.0 ? r2 : 0.0);
             }
         }
@@ -308,11 +344,18 @@ __global__ __launch_bounds__(256) void sup_fused_kernel(const double* __restrict
 }
 
 template <int G>
-void launch_fused(const double* xyz, int n, int L, const double* ref_c, const double* info, double* rot,
+void launch_fused(const double* xyz, int n, int L, const double* ref, double* ref_c, double* info, double* rot,
                   double* trans, double* rmsd, double* out, hipStream_t s)
 {
     constexpr int C = 256 / G;
-    sup_fused_kernel<G><<<(n + C - 1) / C, 256, 0, s>>>(xyz, n, L, ref_c, info, rot, trans, rmsd, out);
+    if constexpr (G > kSupFoldLanes) sup_ref_kernel<<<1, kSupThreads, 0, s>>>(ref, L, ref_c, info);
+    const double* r = G > kSupFoldLanes ? ref_c : ref;
+    if constexpr (G <= kSupFoldLanes)
+        if (L <= G * kSupFewAtoms) {
+            sup_fused_kernel<G, kSupFewAtoms><<<(n + C - 1) / C, 256, 0, s>>>(xyz, n, L, r, info, rot, trans, rmsd, out);
+            return;
+        }
+    sup_fused_kernel<G, kSupAtoms><<<(n + C - 1) / C, 256, 0, s>>>(xyz, n, L, r, info, rot, trans, rmsd, out);
 }
 
 }  // namespace
@@ -326,17 +369,17 @@ void launch_superpose_ensemble(const double* xyz, int n, int L, const double* re
     double* info = ref_c + 3 * (size_t)L;
     double* cov = info + 8;
     double* rt = cov + 16 * (size_t)n;
-    sup_ref_kernel<<<1, kSupThreads, 0, s>>>(ref, L, ref_c, info);
     if (L <= kSupResidentMax) {
         switch (sup_lanes(L)) {
-        case 16: launch_fused<16>(xyz, n, L, ref_c, info, rot, trans, rmsd, out, s); break;
-        case 32: launch_fused<32>(xyz, n, L, ref_c, info, rot, trans, rmsd, out, s); break;
-        case 64: launch_fused<64>(xyz, n, L, ref_c, info, rot, trans, rmsd, out, s); break;
-        case 128: launch_fused<128>(xyz, n, L, ref_c, info, rot, trans, rmsd, out, s); break;
-        default: launch_fused<256>(xyz, n, L, ref_c, info, rot, trans, rmsd, out, s); break;
+        case 16: launch_fused<16>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
+        case 32: launch_fused<32>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
+        case 64: launch_fused<64>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
+        case 128: launch_fused<128>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
+        default: launch_fused<256>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
         }
         return;
     }
+    sup_ref_kernel<<<1, kSupThreads, 0, s>>>(ref, L, ref_c, info);
     sup_cov_kernel<<<n, kSupThreads, 0, s>>>(xyz, L, ref_c, cov);
     sup_rot_kernel<<<(n + 63) / 64, 64, 0, s>>>(cov, n, L, info, rot, trans, rmsd, out ? rt : nullptr);
     if (out) {

@@ -52,6 +52,16 @@ def test_matches_oracle(gpu_ctx, n, L, seed):
     check_fit(fit, x, ref)
 
 
+@pytest.mark.parametrize("L", [15, 16, 64, 65, 80, 81, 128, 129, 160, 161, 257, 320, 321, 512, 513, 640, 1024, 2049])
+def test_lengths_where_the_split_changes(gpu_ctx, L):
+    """Threads per conformation, atoms per thread and who centres the reference
+    change with the atom count; the last work-group is partly empty, and the
+    reference is far from the origin."""
+    x = B.generate_ensemble(L, 19, L, sigma=(0.5, 3.0))
+    ref = B.generate_ensemble(L + 1, 1, L, sigma=(1.0, 1.0))[0] + np.array([300.0, -200.0, 100.0])
+    check_fit(B.superpose_ensemble(x, reference=ref, ctx=gpu_ctx), x, ref)
+
+
 def test_rigid_copies_land_on_the_reference(gpu_ctx):
     rng = np.random.default_rng(11)
     ref = rng.normal(size=(123, 3)) * 8
