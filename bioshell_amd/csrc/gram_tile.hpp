@@ -54,6 +54,58 @@ __device__ __forceinline__ void solve_pairs(const double (&E)[P][9], const doubl
     }
 }
 
+// The constants of a TILE x TILE tile's rows and columns to LDS, by all the
+// threads of the tile.
+template <int TILE, int THREADS>
+__device__ __forceinline__ void epilogue_consts(const GramArgs& a, int tr, int tc, double* sconst, int tid)
+{
+    for (int v = tid; v < kNumConsts * 2 * TILE; v += THREADS) {
+        const int q = v / (2 * TILE), r = v % (2 * TILE);
+        const bool is_row = r < TILE;
+        const int conf = is_row ? tr * TILE + r : tc * TILE + (r - TILE);
+        const double val = is_row ? (conf < a.n_rows ? a.consts_a[(int64_t)q * a.lda + conf] : 0.0)
+                                  : (conf < a.n_cols ? a.consts_b[(int64_t)q * a.ldb + conf] : 0.0);
+        sconst[r * 12 + q] = val;
+    }
+}
+
+// Folds the keys of a 64 x 64 tile in LDS into its 256 row and column keys at
+// a.stats_part, by the work-group.
+__device__ __forceinline__ void epilogue_fold(const GramArgs& a, int tr, int tc, const unsigned* skeys, int thread)
+{
+    // tile row r and tile column r: four threads of 16 entries each, then two shuffles
+    const int r = thread >> 2, q = thread & 3;
+    unsigned lo = 0xFFFFFFFFu, hi = 0u, clo = 0xFFFFFFFFu, chi = 0u;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const unsigned kr = skeys[r * 65 + q * 16 + c];
+        const unsigned kc = skeys[(q * 16 + c) * 65 + r];
+        lo = min(lo, kr);
+        hi = max(hi, kr == 0xFFFFFFFFu ? 0u : kr);
+        clo = min(clo, kc);
+        chi = max(chi, kc == 0xFFFFFFFFu ? 0u : kc);
+    }
+#pragma unroll
+    for (int m = 1; m <= 2; m <<= 1) {
+        lo = min(lo, (unsigned)__shfl_xor((int)lo, m));
+        hi = max(hi, (unsigned)__shfl_xor((int)hi, m));
+        clo = min(clo, (unsigned)__shfl_xor((int)clo, m));
+        chi = max(chi, (unsigned)__shfl_xor((int)chi, m));
+    }
+    if (q == 0) {
+        const int64_t b = (int64_t)tr * a.stats_T - (int64_t)tr * (tr - 1) / 2 + (tc - tr);
+        unsigned* out = a.stats_part + b * (256 * a.stats_banks);
+        out[r] = lo;
+        out[64 + r] = hi;
+        out[128 + r] = clo;
+        out[192 + r] = chi;
+        if (a.stats_banks == 2) {
+            out[256 + r] = out[384 + r] = 0xFFFFFFFFu;
+            out[320 + r] = out[448 + r] = 0u;
+        }
+    }
+}
+
 // The FP64 QCP epilogue of a TILE x TILE tile whose accumulators the calling
 // waves hold: TILE 64 is four waves of a work-group (wave w owns rows
 // 32 (w/2) .. +31 and columns 32 (w%2) .. +31), TILE 32 is one wave on its own.
@@ -88,14 +140,7 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
     const int wr = wv >> 1, wc = wv & 1;
     double* sconst = reinterpret_cast<double*>(lds);
     if constexpr (kWaves == 1) wave_lds_sync();  // earlier reads of this region are done
-    for (int v = tid; v < kNumConsts * 2 * TILE; v += kThreads) {
-        const int q = v / (2 * TILE), r = v % (2 * TILE);
-        const bool is_row = r < TILE;
-        const int conf = is_row ? tr * TILE + r : tc * TILE + (r - TILE);
-        const double val = is_row ? (conf < a.n_rows ? a.consts_a[(int64_t)q * a.lda + conf] : 0.0)
-                                  : (conf < a.n_cols ? a.consts_b[(int64_t)q * a.ldb + conf] : 0.0);
-        sconst[r * 12 + q] = val;
-    }
+    epilogue_consts<TILE, kThreads>(a, tr, tc, sconst, tid);
     if constexpr (kWaves == 1)
         wave_lds_sync();
     else
@@ -160,37 +205,7 @@ __device__ __forceinline__ void epilogue(const GramArgs& a, int tr, int tc, f32x
     });
     if constexpr (STATS) {
         __syncthreads();  // every wave's keys are in LDS
-        // tile row r and tile column r: four threads of 16 entries each, then two shuffles
-        const int r = thread >> 2, q = thread & 3;
-        unsigned lo = 0xFFFFFFFFu, hi = 0u, clo = 0xFFFFFFFFu, chi = 0u;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const unsigned kr = skeys[r * 65 + q * 16 + c];
-            const unsigned kc = skeys[(q * 16 + c) * 65 + r];
-            lo = min(lo, kr);
-            hi = max(hi, kr == 0xFFFFFFFFu ? 0u : kr);
-            clo = min(clo, kc);
-            chi = max(chi, kc == 0xFFFFFFFFu ? 0u : kc);
-        }
-#pragma unroll
-        for (int m = 1; m <= 2; m <<= 1) {
-            lo = min(lo, (unsigned)__shfl_xor((int)lo, m));
-            hi = max(hi, (unsigned)__shfl_xor((int)hi, m));
-            clo = min(clo, (unsigned)__shfl_xor((int)clo, m));
-            chi = max(chi, (unsigned)__shfl_xor((int)chi, m));
-        }
-        if (q == 0) {
-            const int64_t b = (int64_t)tr * a.stats_T - (int64_t)tr * (tr - 1) / 2 + (tc - tr);
-            unsigned* out = a.stats_part + b * (256 * a.stats_banks);
-            out[r] = lo;
-            out[64 + r] = hi;
-            out[128 + r] = clo;
-            out[192 + r] = chi;
-            if (a.stats_banks == 2) {
-                out[256 + r] = out[384 + r] = 0xFFFFFFFFu;
-                out[320 + r] = out[448 + r] = 0u;
-            }
-        }
+        epilogue_fold(a, tr, tc, skeys, thread);
     }
 }
 
@@ -409,6 +424,40 @@ __device__ __forceinline__ void gram_tile64(const GramArgs& a, int tr, int tc,
         }                                                                         \
         BS_WAIT_LDS0();                                                           \
         __builtin_amdgcn_sched_barrier(0);                                        \
+    }
+
+    // A wave whose 32 x 32 pairs are all outside the matrix or below its
+    // diagonal only streams its operand block and its share of the constants,
+    // and leaves the matrix and vector units to the other waves of the CU (in a
+    // batch of 512 ensembles of up to 500 x 800 a fifth of the quadrants: 1477
+    // -> 1440 us).
+    if (tr * 64 + (wvu >> 1) * 32 >= a.n_rows || tc * 64 + (wvu & 1) * 32 >= a.n_cols ||
+        (a.triangle && tr == tc && wvu == 2)) {
+        __builtin_amdgcn_s_setprio(2);
+        BS_ISSUE(0, 0)
+        BS_ISSUE(1, 1)
+        BS_ISSUE(2, 2)
+        BS_WAIT_VMCNT(12);
+        __syncthreads();
+        for (int kb = 0, st = 0; kb < n_kblk; ++kb) {
+            BS_WAIT_VMCNT(6);
+            __builtin_amdgcn_s_barrier();
+            BS_ISSUE(kb + 3, st)
+            st = st == 2 ? 0 : st + 1;
+        }
+        BS_WAIT_VMCNT(0);
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
+        double* sconst = reinterpret_cast<double*>(&lds[0][0][0]);
+        epilogue_consts<64, 256>(a, tr, tc, sconst, thread);
+        __syncthreads();
+        if constexpr (STATS) {
+            unsigned* skeys = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(sconst) + epilogue_lds_bytes<64>());
+            for (int v = lane; v < 1024; v += 64) skeys[(wr * 32 + (v >> 5)) * 65 + wc * 32 + (v & 31)] = 0xFFFFFFFFu;
+            __syncthreads();
+            epilogue_fold(a, tr, tc, skeys, thread);
+        }
+        return;
     }
 
     f32x16 acc[9];
