@@ -69,6 +69,7 @@ void context_release(bs_context* ctx)
             if (ctx->ev_copy[k]) (void)hipEventDestroy(ctx->ev_copy[k]);
         }
         if (ctx->h_blk_counts) (void)hipHostFree(ctx->h_blk_counts);
+        if (ctx->h_pair) (void)hipHostFree(ctx->h_pair);
         if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
         ctx->ws_xyz.reset();
         ctx->ws_out.reset();
@@ -196,6 +197,25 @@ bs_status bs_crmsd_pair_f64(bs_context* ctx, const double* a_xyz, const double* 
         hipStream_t s = ctx->stream;
         double* d = static_cast<double*>(ctx->ws_xyz.ensure(n_atoms * 6 * 8, "pair coordinates"));
         double* o = static_cast<double*>(ctx->ws_out.ensure(64, "pair output"));
+        if (n_atoms <= (size_t)kPairMaxAtoms) {
+            // staged in pinned memory, which the kernel reads and writes itself
+            // (the workspace above still decides what a budget refuses)
+            constexpr size_t kResult = (size_t)kPairMaxAtoms * 6;
+            if (!ctx->h_pair)
+                BS_HIP(hipHostMalloc((void**)&ctx->h_pair, (kResult + 8) * 8, hipHostMallocDefault));
+            double* h = ctx->h_pair;
+            std::memcpy(h, a_xyz, n_atoms * 24);
+            std::memcpy(h + 3 * n_atoms, b_xyz, n_atoms * 24);
+            RunRecord* rec = ctx->begin_record();
+            rec->base.pairs = 1;
+            launch_pair(h, h + 3 * n_atoms, (int)n_atoms, h + kResult, s, rec->clk);
+            BS_HIP(hipGetLastError());
+            rec->kind = RunRecord::kOneStage;
+            rec->base.main_launches = 1;
+            BS_HIP(hipStreamSynchronize(s));
+            *out = h[kResult];
+            return;
+        }
         BS_HIP(hipMemcpyAsync(d, a_xyz, n_atoms * 24, hipMemcpyHostToDevice, s));
         BS_HIP(hipMemcpyAsync(d + 3 * n_atoms, b_xyz, n_atoms * 24, hipMemcpyHostToDevice, s));
         avsa_device(ctx, d, 2, (int)n_atoms, BS_FP64_PLAIN, o, true);

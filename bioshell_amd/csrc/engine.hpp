@@ -238,6 +238,7 @@ struct bs_context {
     void* h_blk[2] = {nullptr, nullptr};  // pinned result blocks
     size_t h_blk_cap = 0;
     uint32_t* h_blk_counts = nullptr;  // pinned flagged counts, one per block
+    double* h_pair = nullptr;          // pinned: one pair's coordinates, then its result
     size_t h_blk_counts_cap = 0;
     hipEvent_t ev_compute[2] = {}, ev_copy[2] = {};
     bs::QueryWorkspace qws;    // synchronous query calls

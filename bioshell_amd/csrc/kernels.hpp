@@ -29,6 +29,10 @@ size_t exact_scratch_bytes(int n, int L, int n_cu);
 bool exact_small(int n, int L, int n_cu);
 void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
                        hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
+// cRMSD of one pair of at most kPairMaxAtoms atoms, FP64, one launch; a, b and
+// out on the device or in pinned host memory.
+constexpr int kPairMaxAtoms = 3072;
+void launch_pair(const double* a, const double* b, int L, double* out, hipStream_t s, uint64_t* clk = nullptr);
 int plain_block(int n, bool fp64, bool alone, int n_cu);
 inline int plain_tiles_per_side(int n, int r) { return (n + 16 * r - 1) / (16 * r); }
 // One ensemble of a batched plain launch (f32 output); nt tiles per side.

@@ -343,7 +343,87 @@ size_t exact_small_lds(int L)
     return (32 * 4 + std::max<size_t>(32 * ((3 * (size_t)L) | 1), 4 * 9 * 256)) * 8;
 }
 
+// ------------------------------------------------------------------ one pair
+// Two conformations of at most 256 kPairAtoms atoms by one work-group, every
+// atom in registers, read once: a and b, like the result, may be pinned host
+// memory, which the copies to and from the device cost more than the reads
+// over the bus do.  Bound by latency: a call for 76 atoms takes 20 us, 39 with
+// two copies in, the tile kernel and a copy out.
+constexpr int kPairAtoms = kPairMaxAtoms / 256;
+
+template <int N>
+__device__ inline void pair_sum(double (&v)[N], double (*part)[11])
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = wave_sum(v[q]);
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < N; ++q) part[w][q] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = (part[0][q] + part[1][q]) + (part[2][q] + part[3][q]);
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void pair_kernel(const double* a, const double* b, int L, double* out,
+                                                   uint64_t* t_start, uint64_t* t_end)
+{
+    __shared__ double part[4][11];
+    stamp_start(t_start);
+    double x[kPairAtoms][6];
+    double c[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < kPairAtoms; ++j) {
+        if (256 * j >= L) break;  // uniform
+        const int k = 3 * min((int)threadIdx.x + 256 * j, L - 1);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            x[j][q] = a[k + q];
+            x[j][3 + q] = b[k + q];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kPairAtoms; ++j) {
+        if (256 * j >= L) break;
+        const bool in = (int)threadIdx.x + 256 * j < L;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) c[q] += in ? x[j][q] : 0.0;
+    }
+    pair_sum<6>(c, part);
+    double v[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // covariance, inner products
+#pragma unroll
+    for (int j = 0; j < kPairAtoms; ++j) {
+        if (256 * j >= L) break;
+        const bool in = (int)threadIdx.x + 256 * j < L;
+        double d[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) d[q] = in ? x[j][q] - c[q] / L : 0.0;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v[3 * p + q] += d[p] * d[3 + q];
+            v[9] += d[p] * d[p];
+            v[10] += d[3 + p] * d[3 + p];
+        }
+    }
+    pair_sum<11>(v, part);
+    if (threadIdx.x < 64) {
+        const double m[9] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]};
+        const double r = exact_rmsd(m, v[9], v[10], L);
+        if (threadIdx.x == 0) {
+            *out = r;
+            if (t_end) *t_end = wall_clock64();
+        }
+    }
+}
+
 }  // namespace
+
+void launch_pair(const double* a, const double* b, int L, double* out, hipStream_t s, uint64_t* clk)
+{
+    pair_kernel<<<1, 256, 0, s>>>(a, b, L, out, clk ? clk + kClkStart : nullptr, clk ? clk + kClkEnd : nullptr);
+}
 
 // One launch while the LDS holds the coordinates (up to 211 atoms) and every
 // work-group is resident at once: a second round costs more than the second

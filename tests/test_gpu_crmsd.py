@@ -43,6 +43,21 @@ def test_pair_fp64(gpu_ctx):
         assert B.crmsd(a, b, ctx=gpu_ctx) == pytest.approx(O.crmsd(a, b), abs=1e-9)
 
 
+@pytest.mark.parametrize("L", [1, 2, 3, 63, 64, 65, 255, 256, 257, 1500, 2816, 2817, 3072, 3073])
+def test_pair_lengths(gpu_ctx, L):
+    """One pair at the edges of its kernel's waves and atoms per thread, and
+    above, far from the origin; and the pair's mirror image and copy.
+    RMSD^2 carries the rounding of (G_a + G_b) / L at that distance."""
+    x = B.generate_ensemble(L, 2, L, sigma=(1.0, 2.0)) + 500.0
+    a, b = x
+    for p, q in ((a, b), (a, a), (a, a * [1, 1, -1] + [0, 0, 1000.0])):
+        want, got = O.crmsd(p, q), B.crmsd(p, q, ctx=gpu_ctx)
+        g = ((p - p.mean(0)) ** 2).sum() + ((q - q.mean(0)) ** 2).sum()
+        d = 1e4 * np.finfo(np.float64).eps * (g / L + 1.0)
+        assert abs(got - want) <= min(np.sqrt(d), d / max(want, 1e-300)) + 1e-9, (got, want)
+    assert gpu_ctx.last_stats()["pairs"] == 1 and gpu_ctx.last_stats()["total_ms"] > 0
+
+
 def test_superpose_fp64(gpu_ctx):
     rng = np.random.default_rng(1)
     a = rng.normal(size=(40, 3)) * 6
