@@ -8,10 +8,11 @@
 // maxima with integer atomics on the float bit patterns (distances are >= 0,
 // whose IEEE patterns order like unsigned integers).
 //
-// The agglomeration follows bioshell-clustering/src/hierarchical/
-// clustering_matrix.rs step for step on a dense f32 matrix in HBM (see the
-// comments at each phase); the merge sequence it records is what the host
-// rebuilds the tree from.
+// The agglomeration, two kernels per merge, for element counts beyond those of
+// the one-launch form (kernels_agglom.hip, up to about 16,000), follows
+// bioshell-clustering/src/hierarchical/clustering_matrix.rs step for step on a
+// dense f32 matrix in HBM (see the comments at each phase); the merge sequence
+// it records is what the host rebuilds the tree from.
 #include "cluster_rule.hpp"
 #include "kernels.hpp"
 #include "wave.hpp"

@@ -1,4 +1,6 @@
-// kernels_plain.hip -- the plain per-pair cRMSD kernel (FP64 and FP32).
+// kernels_plain.hip -- the plain per-pair cRMSD kernel (FP64 and FP32): FP32,
+// batches of both, and FP64 where there is no room for the matrix form's
+// centroids (kernels_exact.hip).
 //
 // Every pair walks the textbook steps: the two centred conformations
 // (centroid = sum / n, then subtract, as in
