@@ -70,6 +70,7 @@ void context_release(bs_context* ctx)
         }
         if (ctx->h_blk_counts) (void)hipHostFree(ctx->h_blk_counts);
         if (ctx->h_pair) (void)hipHostFree(ctx->h_pair);
+        if (ctx->h_query) (void)hipHostFree(ctx->h_query);
         if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
         ctx->ws_xyz.reset();
         ctx->ws_out.reset();

@@ -239,6 +239,7 @@ struct bs_context {
     size_t h_blk_cap = 0;
     uint32_t* h_blk_counts = nullptr;  // pinned flagged counts, one per block
     double* h_pair = nullptr;          // pinned: one pair's coordinates, then its result
+    char* h_query = nullptr;           // pinned: a small call's queries, then its top-k results
     size_t h_blk_counts_cap = 0;
     hipEvent_t ev_compute[2] = {}, ev_copy[2] = {};
     bs::QueryWorkspace qws;    // synchronous query calls

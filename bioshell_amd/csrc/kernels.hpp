@@ -340,6 +340,8 @@ void launch_superpose(const double* a, const double* b, int L, double* out13, hi
 // n x 3, rmsd n and, when out is not null, the superposed n x L x 3.  scratch
 // holds superpose_scratch_bytes(n, L); any of rot / trans / rmsd may be null.
 size_t superpose_scratch_bytes(int n, int L);
+// n doubles from src (pinned host memory, both 16-byte aligned) to dst.
+void launch_copy_doubles(double* dst, const double* src, int64_t n, hipStream_t s);
 void launch_superpose_ensemble(const double* xyz, int n, int L, const double* ref, double* scratch,
                                double* rot, double* trans, double* rmsd, double* out, hipStream_t s);
 

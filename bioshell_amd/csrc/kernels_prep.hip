@@ -121,7 +121,22 @@ __global__ __launch_bounds__(64) void superpose_kernel(const double* __restrict_
     }
 }
 
+__global__ __launch_bounds__(256) void copy_doubles_kernel(double* __restrict__ dst, const double* __restrict__ src,
+                                                           int64_t n)
+{
+    const int64_t v = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+    if (v + 1 < n)
+        *reinterpret_cast<double2*>(dst + v) = *reinterpret_cast<const double2*>(src + v);
+    else if (v < n)
+        dst[v] = src[v];
+}
+
 }  // namespace
+
+void launch_copy_doubles(double* dst, const double* src, int64_t n, hipStream_t s)
+{
+    copy_doubles_kernel<<<(unsigned)((n + 511) / 512), 256, 0, s>>>(dst, src, n);
+}
 
 void launch_prepare(const double* xyz, int n, int L, int n_pad, int n_kblk, GramMode mode, const double* fixed_ref,
                     double* partial, double* ref, double* rot, double* cent, void* panels, double* consts, int ld,

@@ -391,16 +391,15 @@ __global__ __launch_bounds__(kRowThreads) void topk_row_kernel(const float* __re
         }
         if (less) atomicAdd(&rank[i], less);
         __syncthreads();
-        if (tid < m && rank[tid] < (uint32_t)k) {
-            oi[rank[tid]] = (uint32_t)(own & 0xFFFFFFFFu);
-            ov[rank[tid]] = __uint_as_float((uint32_t)(own >> 32));
-        }
+        if (tid < m && rank[tid] < (uint32_t)k) cand[rank[tid]] = own;
+        __syncthreads();
     } else {
         bitonic_sort(cand, P);
-        for (int v = tid; v < k; v += kRowThreads) {
-            oi[v] = (uint32_t)(cand[v] & 0xFFFFFFFFu);
-            ov[v] = __uint_as_float((uint32_t)(cand[v] >> 32));
-        }
+    }
+    // in order: the results may be in host memory, where single words are slow
+    for (int v = tid; v < k; v += kRowThreads) {
+        oi[v] = (uint32_t)(cand[v] & 0xFFFFFFFFu);
+        ov[v] = __uint_as_float((uint32_t)(cand[v] >> 32));
     }
     stamp_end(t_end, done);
 }

@@ -70,13 +70,16 @@ void QueryWorkspace::reserve(int n_q, int n_lib, int L, int k)
 // against the library's reference, Gram + epilogue + FP64 re-evaluation into
 // ws.scores (n_q x n_lib), and, when k > 0, top-k into ws.topk.
 void enqueue_query(bs_library* lib, QueryWorkspace& ws, const double* q_host, int n_q, int k,
-                   hipStream_t s, RunRecord* rec)
+                   hipStream_t s, RunRecord* rec, const QueryStage& stage)
 {
     const int L = lib->P.L, n_lib = lib->P.n;
     double* dq = static_cast<double*>(ws.xyz.ensure((size_t)n_q * L * 3 * 8, "query coordinates"));
     float* scores =
         static_cast<float*>(ws.scores.ensure((size_t)n_q * n_lib * 4, "query scores"));
-    BS_HIP(hipMemcpyAsync(dq, q_host, (size_t)n_q * L * 3 * 8, hipMemcpyHostToDevice, s));
+    if (stage.queries)
+        launch_copy_doubles(dq, stage.queries, (int64_t)n_q * L * 3, s);
+    else
+        BS_HIP(hipMemcpyAsync(dq, q_host, (size_t)n_q * L * 3 * 8, hipMemcpyHostToDevice, s));
     prepare(ws.prep, dq, n_q, L, lib->P.mode, lib->P.ref.as<double>(), s, rec ? rec->clk + kClkStart : nullptr);
     GramRun run;
     if (rec) {
@@ -90,9 +93,10 @@ void enqueue_query(bs_library* lib, QueryWorkspace& ws, const double* q_host, in
     ws.gsc.max_wg = lib->ctx->gsc.max_wg;
     run_gram(view_of(ws.prep), view_of(lib->P), run, ws.gsc, s);
     if (k > 0) {
-        uint32_t* idx = static_cast<uint32_t*>(ws.topk.ensure(topk_bytes(n_q, n_lib, k), "top-k"));
+        uint32_t* own = static_cast<uint32_t*>(ws.topk.ensure(topk_bytes(n_q, n_lib, k), "top-k"));
+        uint32_t* idx = stage.results ? stage.results : own;
         float* val = reinterpret_cast<float*>(idx + (size_t)n_q * k);
-        launch_topk(scores, n_q, n_lib, k, idx, val, idx + (size_t)n_q * k * 2, s,
+        launch_topk(scores, n_q, n_lib, k, idx, val, own + (size_t)n_q * k * 2, s,
                     rec ? rec->clk + kClkEnd : nullptr, rec ? rec->done : nullptr);
         BS_HIP(hipGetLastError());
     }
@@ -163,6 +167,9 @@ void bs_library_destroy(bs_library* lib)
 size_t bs_library_size(const bs_library* lib) { return lib ? (size_t)lib->P.n : 0; }
 size_t bs_library_atoms(const bs_library* lib) { return lib ? (size_t)lib->P.L : 0; }
 
+// Pinned bytes of a context for the queries and results of a small call.
+constexpr size_t kStageQueries = 1 << 20, kStageResults = 256 << 10;
+
 static void check_query(bs_context* ctx, bs_library* lib, const double* q, size_t n_q)
 {
     BS_REQUIRE(ctx != nullptr && lib != nullptr, "null context or library");
@@ -200,6 +207,22 @@ bs_status bs_query_topk(bs_context* ctx, bs_library* lib, const double* q_xyz, s
         BS_HIP(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
         ctx->qws.bind(&ctx->budget);
+        // Small calls go through pinned memory: copies of pageable memory cost
+        // about 15 us each way (32 queries of 256 atoms, k 100: a call 96 -> 83 us).
+        const size_t q_bytes = n_q * lib->P.L * 24, r_bytes = n_q * k * 8;
+        if (q_bytes <= kStageQueries && r_bytes <= kStageResults) {
+            if (!ctx->h_query)
+                BS_HIP(hipHostMalloc((void**)&ctx->h_query, kStageQueries + kStageResults, hipHostMallocDefault));
+            QueryStage stage;
+            stage.queries = reinterpret_cast<const double*>(ctx->h_query);
+            stage.results = reinterpret_cast<uint32_t*>(ctx->h_query + kStageQueries);
+            std::memcpy(ctx->h_query, q_xyz, q_bytes);
+            enqueue_query(lib, ctx->qws, q_xyz, (int)n_q, (int)k, s, ctx->begin_record(), stage);
+            BS_HIP(hipStreamSynchronize(s));
+            std::memcpy(idx, stage.results, n_q * k * 4);
+            std::memcpy(rmsd, stage.results + n_q * k, n_q * k * 4);
+            return;
+        }
         enqueue_query(lib, ctx->qws, q_xyz, (int)n_q, (int)k, s, ctx->begin_record());
         const uint32_t* d_idx = ctx->qws.topk.as<uint32_t>();
         const float* d_val = reinterpret_cast<const float*>(d_idx + n_q * k);

@@ -110,6 +110,22 @@ def test_topk_row_sizes(gpu_ctx, n, k, copies):
     lib.close()
 
 
+@pytest.mark.parametrize("n,L,n_q,k", [(300, 33, 1, 5), (300, 700, 62, 100), (300, 700, 63, 100), (1000, 20, 32, 1000),
+                                       (1100, 20, 33, 1000)])
+def test_topk_call_sizes(gpu_ctx, n, L, n_q, k):
+    """Calls on both sides of what is staged in pinned memory (1 MiB of queries,
+    256 KiB of results), and an odd number of coordinates."""
+    x = B.generate_ensemble(n + L, n + n_q, L, sigma=(0.5, 3.0))
+    lib = B.Library(x[:n], ctx=gpu_ctx)
+    scores = lib.query_all(x[n:])
+    idx, val = lib.query_topk(x[n:], k)
+    for r in range(n_q):
+        order = np.argsort(scores[r], kind="stable")[:k]
+        assert np.array_equal(idx[r], order)
+        assert np.array_equal(val[r], scores[r][order])
+    lib.close()
+
+
 def test_topk_argument_errors(gpu_ctx, bucket):
     lib_x, q, _ = bucket
     lib = B.Library(lib_x[:50], ctx=gpu_ctx)
