@@ -22,7 +22,9 @@ static __device__ __attribute__((noinline)) double exact_polish(double m0, doubl
 // root of the sum of the products' squares), which for pairs that fit badly is
 // far nearer: 3 to 4 steps instead of 6 to 10, and no pair is polished only
 // for its number of steps.  And the step's quotient is rcp with two refinements.
-__device__ inline double exact_rmsd(const double (&m)[9], double gi, double gj, int L)
+// A lane that is not live (its sums are zeros, which would ask for the polish)
+// returns anything.
+__device__ inline double exact_rmsd(const double (&m)[9], double gi, double gj, int L, bool live = true)
 {
     double f2 = 0.0;
 #pragma unroll
@@ -51,7 +53,7 @@ __device__ inline double exact_rmsd(const double (&m)[9], double gi, double gj, 
         if (fabs(step) <= 1e-11 * fabs(l)) break;
     }
     const double scale = fabs(4.0 * l * l * l) + fabs(2.0 * c2 * l) + fabs(c1);
-    if (it > 8 || !(fabs(dp) > 1e-4 * scale)) l = exact_polish(m[0], m[1], m[2], m[3], m[4], m[5], m[6], m[7], m[8]);
+    if (live & ((it > 8) | !(fabs(dp) > 1e-4 * scale))) l = exact_polish(m[0], m[1], m[2], m[3], m[4], m[5], m[6], m[7], m[8]);
     const double r2 = 2.0 * (E0 - l) / L;
     return sqrt(r2 > 0.0 ? r2 : 0.0);
 }

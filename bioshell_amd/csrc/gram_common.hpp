@@ -233,7 +233,7 @@ __device__ inline double fallback_pairs(const PairRef& p, int lane)
         mine.ga = keep ? va : mine.ga;
         mine.gb = keep ? vb : mine.gb;
     }
-    return exact_rmsd(mine.m, mine.ga, mine.gb, max(p.L, 1));
+    return exact_rmsd(mine.m, mine.ga, mine.gb, max(p.L, 1), p.L > 0);
 }
 
 // Walks a wave through the flagged outputs, up to 64 at a time: its share of
