@@ -13,8 +13,11 @@
 // (rotation_fast, Newton from E0 = (G_x + G_r) / 2) and the RMSD, and every
 // thread writes R x + t for its atoms.  Every wave centres the reference for
 // itself, while its conformations are on their way; above 512 atoms, where
-// that is many loads a lane, one block does so in a launch before.  Chains
-// longer than 2048 atoms take three passes (covariance per block, Jacobi per thread, apply per atom).
+// that is many loads a lane, one block does so in a launch before.  A reference
+// that lies in one of the outputs (a row of the last call's coordinates, whose
+// buffer this call fills again) is copied to the scratch before anything is
+// written.  Chains longer than 2048 atoms take three passes (covariance per
+// block, Jacobi per thread, apply per atom).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -167,6 +170,13 @@ __global__ __launch_bounds__(256) void sup_apply_kernel(const double* __restrict
     }
 }
 
+// n doubles of a reference to the scratch, by one block.
+__global__ __launch_bounds__(kSupThreads) void sup_copy_kernel(const double* __restrict__ src, int n,
+                                                               double* __restrict__ dst)
+{
+    for (int k = threadIdx.x; k < n; k += kSupThreads) dst[k] = src[k];
+}
+
 // ---------------------------------------------------------------- fused form
 constexpr int kSupAtoms = 8;                 // atoms per thread held in registers, at most
 // With at most this many a fourth work-group fits on a CU (10,000 x 300: 42.6 ->
@@ -191,7 +201,8 @@ struct SupLds {
     double rc[3];       // the reference's centroid
 };
 
-// ref: the reference itself (G <= kSupFoldLanes), else its centred copy, with
+// ref: the reference itself (G <= kSupFoldLanes), which no output may overlap
+// (every work-group reads it while others write), else its centred copy, with
 // its centroid at info.  Bound by memory: 10,000 x 300 is 144 MB (28 us at a
 // copy's rate) in 40 us, 42 with the reference centred by a launch of its own,
 // 3000 x 120 in 9 and 12.
@@ -370,6 +381,16 @@ void launch_superpose_ensemble(const double* xyz, int n, int L, const double* re
     double* cov = info + 8;
     double* rt = cov + 16 * (size_t)n;
     if (L <= kSupResidentMax) {
+        auto meets = [&](const double* p, size_t count) {
+            const auto r = reinterpret_cast<uintptr_t>(ref), o = reinterpret_cast<uintptr_t>(p);
+            return p && r < o + count * 8 && o < r + (size_t)L * 24;
+        };
+        if (sup_lanes(L) <= kSupFoldLanes &&
+            (meets(rot, 9 * (size_t)n) || meets(trans, 3 * (size_t)n) || meets(rmsd, n) ||
+             meets(out, 3 * (size_t)n * L))) {
+            sup_copy_kernel<<<1, kSupThreads, 0, s>>>(ref, 3 * L, ref_c);
+            ref = ref_c;
+        }
         switch (sup_lanes(L)) {
         case 16: launch_fused<16>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;
         case 32: launch_fused<32>(xyz, n, L, ref, ref_c, info, rot, trans, rmsd, out, s); break;

@@ -155,8 +155,9 @@ bs_status bs_superpose_ensemble(bs_context* ctx, const double* xyz, size_t n_con
                                 const double* ref_xyz, size_t ref_index, double* rot9,
                                 double* trans3, double* rmsd, double* superposed);
 /* The same on device buffers, asynchronous on the context's stream; d_ref may
- * be NULL (conformation ref_index is the reference); d_superposed must not
- * overlap d_xyz. */
+ * be NULL (conformation ref_index is the reference) and may lie in an output
+ * buffer (a row of an earlier call's d_superposed): it is read before anything
+ * is written.  d_superposed must not overlap d_xyz. */
 bs_status bs_superpose_ensemble_device(bs_context* ctx, const double* d_xyz, size_t n_conf,
                                        size_t n_atoms, const double* d_ref, size_t ref_index,
                                        double* d_rot9, double* d_trans3, double* d_rmsd,

@@ -125,6 +125,41 @@ def test_device_entry_matches_host(gpu_ctx):
     assert np.array_equal(d_sp.cpu().numpy(), host.superposed)
 
 
+@pytest.mark.parametrize("where", ["superposed", "rotations", "rmsd"])
+@pytest.mark.parametrize("L", [16, 80, 300, 512, 513, 2049])
+def test_reference_in_an_output_buffer(gpu_ctx, L, where):
+    """Iterated fitting onto a row of the last pass's coordinates, with the same
+    buffer filled again: the reference is read before anything is written, at
+    every length (short chains read it in the launch that writes).  More
+    work-groups than the device holds at once, and the reference where the
+    first of them write."""
+    import torch
+
+    n = 17600 if L <= 128 else max(4400, 3 * L)
+    x = B.generate_ensemble(L, n, L, sigma=(0.5, 3.0))
+    ref = B.generate_ensemble(L + 1, 1, L, sigma=(1.0, 1.0))[0] + np.array([30.0, -20.0, 10.0])
+    d_x = torch.from_numpy(x).cuda()
+
+    def fit(d_ref):
+        out = dict(rotations=torch.zeros((n, 9), dtype=torch.float64, device="cuda"),
+                   translations=torch.zeros((n, 3), dtype=torch.float64, device="cuda"),
+                   rmsd=torch.zeros(n, dtype=torch.float64, device="cuda"),
+                   superposed=torch.zeros((n, L, 3), dtype=torch.float64, device="cuda"))
+        if d_ref is None:
+            d_ref = out[where].view(-1)[:3 * L]
+        d_ref.copy_(torch.from_numpy(ref.ravel()))
+        torch.cuda.synchronize()
+        B.superpose_ensemble_device(d_x.data_ptr(), n, L, d_ref.data_ptr(), 0, *(o.data_ptr() for o in out.values()),
+                                    ctx=gpu_ctx)
+        gpu_ctx.synchronize()
+        return out
+
+    want = fit(torch.empty(3 * L, dtype=torch.float64, device="cuda"))
+    got = fit(None)
+    for k in want:
+        assert torch.equal(got[k], want[k]), k
+
+
 def test_file_to_superposed_pdb(gpu_ctx, golden_2jqb, tmp_path):
     """2jqb read natively, cRMSD against the numpy-SVD golden values, every
     model fitted onto model 0, written as PDB and read back."""
