@@ -320,7 +320,7 @@ struct AgglomArgs {
     float* md;
     uint64_t* slots;
     float* newrow;
-    unsigned* status;       // set when a wait ran into max_wait
+    unsigned* status;       // set when a wait ran into max_wait: the merges are incomplete
     uint64_t max_wait;      // ticks of the wall clock
     int rows, n_blocks, block_shift;  // filled by launch_agglom from the plan
 };

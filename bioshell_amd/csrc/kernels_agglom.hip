@@ -235,8 +235,8 @@ __global__ __launch_bounds__(64 * kWaves) void agglom_kernel(AgglomArgs a)
                 const uint64_t* q = a.slots + (size_t)(s % 3) * G + t;
                 const uint64_t t0 = wall_clock64();
                 int spin = 0;
-                while ((k = agent_load(q)) == 0ull) {
-                    if ((++spin & 255) == 0 && wall_clock64() - t0 > a.max_wait) {
+                while ((k = agent_load(q)) == 0ull || a.max_wait == 0) {  // 0: gives up at once
+                    if (a.max_wait == 0 || ((++spin & 255) == 0 && wall_clock64() - t0 > a.max_wait)) {
                         ctl[0] = 1u;
                         break;
                     }

@@ -295,3 +295,17 @@ def test_large_single_link_heights(gpu_ctx, n):
     up = np.concatenate([np.abs(y[i] - y[i + 1:]) for i in range(n - 1)])
     _, _, md = device_merges(gpu_ctx, up, n, "single")
     assert np.array_equal(md, np.sort(np.diff(x)))
+
+
+@pytest.mark.parametrize("linkage", C.LINKAGES)
+@pytest.mark.parametrize("n,kind", [(2, "uniform"), (3, "ties"), (65, "ties"), (300, "euclid"), (700, "ties")])
+def test_launch_that_gives_up_leaves_the_call_to_the_stepwise_loop(gpu_ctx, monkeypatch, linkage, n, kind):
+    """The one-launch loop's work-groups wait for each other up to a limit.  At
+    the limit (0 here: they give up at the first exchange) the call does not
+    fail: the stepwise kernels run it, with the oracle's merges."""
+    up = random_upper(np.random.default_rng(n + len(kind)), n, kind)
+    monkeypatch.setenv("BIOSHELL_CLUSTER_MAX_WAIT_MS", "0")
+    got = device_merges(gpu_ctx, up, n, linkage)
+    want = O.hclust(up, n, linkage)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
