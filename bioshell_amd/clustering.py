@@ -69,25 +69,41 @@ class ClusteringTreeNode:
             nd.left, nd.right = nd.right, nd.left
 
 
+def _python_numbers(values, kinds: str, convert):
+    """The values as Python numbers: at once from arrays of the given dtype
+    kinds, else converted one by one."""
+    a = np.asarray(values)
+    return a.tolist() if a.dtype.kind in kinds else [convert(v) for v in a.tolist()]
+
+
 def tree_from_merges(n: int, merge_i, merge_j, merge_d) -> ClusteringTreeNode:
     """Replays a merge sequence with the reference's index bookkeeping: the
     merged cluster takes index i, the last active cluster moves to index j
-    (hierarchical.rs:44-78)."""
+    (hierarchical.rs:44-78).  An index that names no active cluster, as in a
+    merge of two equal ones, is a KeyError."""
     if n < 1:
         raise ValueError("nothing to cluster")
     # Python numbers and a list, not numpy scalars and a dict: 10,000 elements
     # take 14 ms instead of 21
-    merges = zip(np.asarray(merge_i).tolist(), np.asarray(merge_j).tolist(), np.asarray(merge_d).tolist())
+    mi, mj = _python_numbers(merge_i, "iu", int), _python_numbers(merge_j, "iu", int)
+    md = _python_numbers(merge_d, "f", float)
+    m = min(len(mi), len(mj), len(md))
+    lowest = min(min(mi[:m], default=0), min(mj[:m], default=0))
+    if lowest < 0:  # a list would count from its end
+        raise KeyError(lowest)
     node = ClusteringTreeNode
     clusters = [node(i, 1, 0.0) for i in range(n)]
-    for new_id, (i, j, d) in enumerate(merges, n):
-        if i == j:
-            raise KeyError(j)
-        ci, cj = clusters[i], clusters[j]
-        clusters[i] = node(new_id, ci.cluster_size + cj.cluster_size, d, ci, cj)
-        last = clusters.pop()
-        if j < len(clusters):
-            clusters[j] = last
+    try:
+        for new_id, (i, j, d) in enumerate(zip(mi, mj, md), n):
+            if i == j:
+                raise KeyError(j)
+            ci, cj = clusters[i], clusters[j]
+            clusters[i] = node(new_id, ci.cluster_size + cj.cluster_size, d, ci, cj)
+            last = clusters.pop()
+            if j < len(clusters):
+                clusters[j] = last
+    except IndexError:
+        raise KeyError(max(i, j)) from None
     return clusters[0]
 
 

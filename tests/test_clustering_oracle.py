@@ -284,3 +284,23 @@ def test_row_stats_oracle():
     lo, hi = O.row_stats(up, n)
     assert np.array_equal(lo, np.nanmin(D, axis=1))
     assert np.array_equal(hi, np.nanmax(D, axis=1))
+
+
+@pytest.mark.parametrize("mi,mj", [([0, -1], [1, 0]), ([0, 0], [1, -1]), ([0, 0], [-2, 1]), ([0, 0], [3, 1]),
+                                   ([5, 0], [1, 1]), ([0, 0], [1, 2]), ([0, 0, 0], [2, 1, 0]), ([0, 0, 0], [2, 1, 1])])
+def test_tree_refuses_indices_of_no_cluster(mi, mj):
+    """Negative indices, indices past the active clusters and one merge too
+    many: three elements, two merges at most."""
+    with pytest.raises(KeyError):
+        C.tree_from_merges(3, mi, mj, [1.0, 2.0, 3.0][:len(mi)])
+
+
+def test_tree_from_other_number_types():
+    """Any iterables of numbers: the tree is that of the integer arrays."""
+    mi, mj, md = [0, 0, 0], [3, 1, 1], [1, 2, 3]
+    want = C.tree_from_merges(4, np.array(mi, np.uint32), np.array(mj, np.uint32), np.array(md, np.float32))
+    for make in (lambda v: [float(x) for x in v], lambda v: (x for x in v), lambda v: np.array(v, np.float64),
+                 lambda v: tuple(np.int64(x) for x in v)):
+        root = C.tree_from_merges(4, make(mi), make(mj), make(md))
+        assert C.retrieve_data_id(root) == C.retrieve_data_id(want)
+        assert type(root.merging_distance) is float and root.merging_distance == 3.0
