@@ -126,8 +126,10 @@ bs_run_stats RunRecord::read() const
     bs_run_stats st = base;
     if (kind == kUntimed) return st;
     uint64_t t[kClkWords];
+    // on the context's stream: a plain hipMemcpy would also wait for the null
+    // stream's work, which is none of the context's
+    BS_HIP(hipMemcpyAsync(t, clk, sizeof(t), hipMemcpyDeviceToHost, stream));
     BS_HIP(hipStreamSynchronize(stream));
-    BS_HIP(hipMemcpy(t, clk, sizeof(t), hipMemcpyDeviceToHost));
     auto ms = [&](int a, int b) { return t[b] > t[a] ? (double)(t[b] - t[a]) / khz : 0.0; };
     st.total_ms = ms(kClkStart, kClkEnd);
     if (kind == kOneStage) st.main_ms = st.total_ms;

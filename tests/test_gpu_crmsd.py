@@ -487,3 +487,24 @@ def test_fp64_without_budget():
         ctx.synchronize()
         assert ctx.bytes_in_use() == 0
     assert np.abs(out.cpu().numpy() - O.all_vs_all(x, nthreads=8)).max() <= 1e-5
+
+
+def test_stats_wait_for_the_context_alone(gpu_ctx):
+    """Reading a call's times waits for the context's stream, not for other work
+    on the device: the null stream is still busy when they come back."""
+    import torch
+
+    x = B.generate_ensemble(5, 100, 40, sigma=(0.5, 3.0))
+    B.crmsd_all_vs_all(x, B.Method.BF16X3_GRAM, ctx=gpu_ctx)
+    a = torch.zeros((8192, 8192), dtype=torch.bfloat16, device="cuda")
+    b = torch.zeros_like(a)
+    torch.mm(a, a, out=b)
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    for _ in range(300):  # some 200 ms on the null stream
+        torch.mm(a, a, out=b)
+    done.record()
+    st, hist = gpu_ctx.last_stats(), gpu_ctx.history(3)
+    busy = not done.query()
+    torch.cuda.synchronize()
+    assert busy and st["pairs"] == 100 * 99 // 2 and st["total_ms"] > 0 and len(hist) >= 1
