@@ -36,6 +36,7 @@ void* Budget::alloc(size_t bytes, const char* what)
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here: the caller may go on without this memory
         std::lock_guard<std::mutex> g(mu_);
         used_ -= bytes;
         fail(e == hipErrorOutOfMemory ? BS_ERR_OUT_OF_BUDGET : BS_ERR_HIP, "%s: hipMalloc(%zu) failed: %s",

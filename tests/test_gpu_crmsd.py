@@ -508,3 +508,20 @@ def test_stats_wait_for_the_context_alone(gpu_ctx):
     busy = not done.query()
     torch.cuda.synchronize()
     assert busy and st["pairs"] == 100 * 99 // 2 and st["total_ms"] > 0 and len(hist) >= 1
+
+
+@pytest.mark.parametrize("method", list(B.Method))
+def test_failed_allocation_is_reported_once(method):
+    """An ensemble that no device holds (2^21 x 2^20 atoms, 53 TB) is refused
+    before its coordinates are read, and the thread's next call, which checks
+    its launches, does not report that refusal as its own.  (FP64 goes on
+    without its workspace after such a refusal.)"""
+    import ctypes
+
+    x = B.generate_ensemble(5, 600, 40, sigma=(0.5, 3.0))
+    with B.Context(0) as ctx:
+        want = B.crmsd_all_vs_all(x, method, ctx=ctx).upper
+        word = np.zeros(8)
+        assert B._native.lib().bs_crmsd_all_vs_all(ctx.handle, word.ctypes.data_as(B._native.c_dp), 1 << 21, 1 << 20,
+                                                   int(method), word.ctypes.data_as(ctypes.c_void_p), 1) == -4
+        assert np.array_equal(B.crmsd_all_vs_all(x, method, ctx=ctx).upper, want)
