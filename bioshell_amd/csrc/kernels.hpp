@@ -22,6 +22,10 @@ namespace bs {
 // zero word.
 void launch_plain_avsa(const double* xyz, int n, int L, bool fp64, void* out, bool out_f64,
                        int n_cu, hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
+// Sets the LDS limits of the kernels whose launches choose their size, on the
+// current device; before the first launch there.
+void exact_init();
+void agglom_init();
 // FP64 over one ensemble with the covariance on the matrix unit
 // (kernels_exact.hip); scratch holds exact_scratch_bytes (0 for the small
 // ensembles that take one launch).

@@ -564,14 +564,21 @@ const void* agglom_entry(int rule)
 }
 }  // namespace
 
+// As exact_init; where the limit is not taken the launch is refused.
+void agglom_init()
+{
+    for (int rule = 0; rule < 6; ++rule)
+        for (const void* f : {agglom_entry<false>(rule), agglom_entry<true>(rule)})
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
+                (void)hipGetLastError();
+}
+
 hipError_t launch_agglom(const AgglomPlan& p, AgglomArgs a, hipStream_t s)
 {
     a.rows = p.rows;
     a.n_blocks = p.n_blocks;
     a.block_shift = p.block_shift;
     const void* f = p.block_shift == 6 ? agglom_entry<false>(a.rule) : agglom_entry<true>(a.rule);
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
-    if (e != hipSuccess) return e;
     void* args[] = {&a};
     return hipLaunchCooperativeKernel(f, dim3(p.groups), dim3(64 * kWaves), args, (unsigned)p.lds, s);
 }

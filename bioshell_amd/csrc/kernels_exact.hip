@@ -437,6 +437,15 @@ bool exact_small(int n, int L, int n_cu)
     return lds <= kLdsBytes && nt * (nt + 1) / 2 <= (int64_t)(kLdsBytes / lds) * n_cu;
 }
 
+// The limit is the kernel's, for every thread and context: set once to the
+// most any launch asks for, never to the size of one of them, which another
+// thread's launch may already exceed.
+void exact_init()
+{
+    BS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&exact_small_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
+}
+
 size_t exact_scratch_bytes(int n, int L, int n_cu) { return exact_small(n, L, n_cu) ? 0 : (size_t)n * 32; }
 
 void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
@@ -448,8 +457,6 @@ void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64,
     if (exact_small(n, L, n_cu)) {
         const int nt = (n + 15) / 16, grid = nt * (nt + 1) / 2;
         const int lds = (int)exact_small_lds(L);
-        BS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&exact_small_kernel),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         exact_small_kernel<<<grid, kExactThreads, lds, s>>>(xyz, n, L, nt, out, f, t0, t1, done);
         return;
     }

@@ -525,3 +525,41 @@ def test_failed_allocation_is_reported_once(method):
         assert B._native.lib().bs_crmsd_all_vs_all(ctx.handle, word.ctypes.data_as(B._native.c_dp), 1 << 21, 1 << 20,
                                                    int(method), word.ctypes.data_as(ctypes.c_void_p), 1) == -4
         assert np.array_equal(B.crmsd_all_vs_all(x, method, ctx=ctx).upper, want)
+
+
+def test_two_contexts_with_launches_of_different_lds_sizes():
+    """Two threads, a context each: FP64 ensembles whose launches take 162 KB and
+    75 KB of LDS (the kernel's limit is one for the process), and clusterings,
+    whose work-groups have to be resident together."""
+    import threading
+
+    from bioshell_amd import clustering as C
+
+    shapes = [(64, 211, 260), (33, 8, 1100)]
+    want, got, errors = [], [None, None], []
+    with B.Context(0) as a, B.Context(0) as b:
+        xs = [B.generate_ensemble(n, n, L, sigma=(0.5, 3.0)) for n, L, _ in shapes]
+        ms = [B.crmsd_all_vs_all(B.generate_ensemble(c, c, 30, sigma=(0.5, 3.0)), ctx=a) for _, _, c in shapes]
+        for x, m in zip(xs, ms):
+            want.append((B.crmsd_all_vs_all(x, B.Method.FP64_PLAIN, out_f64=True, ctx=a).upper,
+                         C.retrieve_data_id(C.hierarchical_clustering(m, linkage="average", ctx=a))))
+
+        def work(t, ctx):
+            try:
+                ok = True
+                for r in range(300):
+                    ok &= np.array_equal(B.crmsd_all_vs_all(xs[t], B.Method.FP64_PLAIN, out_f64=True, ctx=ctx).upper,
+                                         want[t][0])
+                    if r % 30 == 0:
+                        tree = C.hierarchical_clustering(ms[t], linkage="average", ctx=ctx)
+                        ok &= C.retrieve_data_id(tree) == want[t][1]
+                got[t] = ok
+            except Exception as e:  # shown by the assertion below
+                errors.append(repr(e))
+
+        th = [threading.Thread(target=work, args=(t, c)) for t, c in enumerate((a, b))]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    assert not errors and got == [True, True]
