@@ -313,7 +313,7 @@ void launch_cluster_step(float* D, int n, int ld, void* state, void* part, int n
                          int rule, unsigned* mi, unsigned* mj, float* md, hipStream_t s);
 
 // The same loop in one launch (kernels_agglom.hip), for the element counts
-// agglom_plan takes (about 15,000 on 256 CUs; the stepwise launches above run
+// agglom_plan takes (up to 16,384 on 256 CUs; the stepwise launches above run
 // the larger ones).  slots (3 x groups), newrow (3 x ld) and status are the
 // exchange buffers; slots and status are zero at the launch.
 struct AgglomArgs {

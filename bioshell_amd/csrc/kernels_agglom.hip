@@ -1,6 +1,6 @@
 // kernels_agglom.hip -- the whole agglomeration loop of hierarchical
-// clustering in one cooperative launch, for the element counts whose caches
-// fit the LDS (about 15,000 on 256 CUs).
+// clustering in one cooperative launch, for up to 16,384 elements (labels of 14
+// bits; the caches then fit the LDS of 224 CUs).
 //
 // The loop is the reference's (clustering_matrix.rs; the rules of the merge,
 // of the move and of ties are listed in kernels_cluster.hip), and its merge
@@ -32,9 +32,9 @@
 //
 // Bound: latency.  Of 4.2 us per merge at 300 elements (12 work-groups) about
 // 1.3 us are the exchange and the rest the dependent steps of one wave, of 7.1
-// us at 10,000 (256 work-groups) about 3.4; memory traffic is below 0.5 TB/s.
+// us at 10,000 (224 work-groups) about 3.4; memory traffic is below 0.5 TB/s.
 // Against two launches per merge: 300 elements 3.2 -> 1.3 ms, 2000 20 -> 10.5
-// ms, 10,000 190 -> 72 ms (average linkage).  Measured and not kept: one
+// ms, 10,000 190 -> 72 ms, 16,300 560 -> 240 ms (average linkage).  Measured and not kept: one
 // work-group without the exchange (as fast up to 180 elements, slower above),
 // the matrix in LDS (3 % at 300 to 2000 elements), 8 waves per work-group (a
 // step is bound by the instructions of its waves).
@@ -518,19 +518,26 @@ __global__ __launch_bounds__(256) void agglom_init_kernel(const float* __restric
 
 }  // namespace
 
-// Work-groups: one per kRowsWanted rows while there are CUs (300 elements:
-// 1.28 ms with 8, 1.24 with 16, 1.31 with 32; 1000: 5.1 with 16, 4.7 with 32,
-// 5.0 with 128; above 6000 every CU has one).  Blocks are 64 columns (one
+// Work-groups: one per kRowsWanted rows (300 elements: 1.28 ms with 8, 1.24
+// with 16, 1.31 with 32; 1000: 5.1 with 16, 4.7 with 32, 5.0 with 128) while
+// there are CUs, of which one in eight is left to others: a work-group's LDS (134 KB
+// at 10,000 elements) keeps most other kernels off its CU until the loop ends,
+// and a launch goes to every shader engine (8 CUs) in turn, so with less than
+// one CU of each free it waits.  An all-vs-all of 400 x 100 in another context,
+// 45 us alone, took up to 71 ms beside 10,000 elements on 256 or 232 CUs and
+// takes up to 0.2 on 224, which costs the loop 1 % (71.5 -> 72.2 ms; 12,100
+// elements 98.3 -> 100.6, 15,200 165 -> 172; 15,800, whose blocks widen for it,
+// 174 -> 240).  Blocks are 64 columns (one
 // 16-byte load of 16 lanes), wider only where the cached minima would not fit
-// the LDS: 128 from about 12,000 elements.
+// the LDS: 128 from 11,201 elements, 256 from 13,557, 512 from 15,617.
 bool agglom_plan(int n, int n_cu, AgglomPlan* out)
 {
     if (n < 2 || n > kMaxElements) return false;
     AgglomPlan p;
-    p.groups = std::max(1, std::min(std::min(n_cu, 64 * kWaves), n / kRowsWanted));
+    p.groups = std::max(1, std::min(std::min(n_cu - n_cu / 8, 64 * kWaves), n / kRowsWanted));
     p.rows = (n + p.groups - 1) / p.groups;
     if (p.rows > 64 * kWaves) return false;
-    for (p.block_shift = 6; p.block_shift <= 8; ++p.block_shift) {
+    for (p.block_shift = 6; p.block_shift <= 9; ++p.block_shift) {
         p.n_blocks = (n + (1 << p.block_shift) - 1) >> p.block_shift;
         const size_t n4 = (size_t)(n + 3) / 4 * 4, cap = (size_t)p.n_blocks << p.block_shift;
         p.lds = (size_t)p.rows * p.n_blocks * 8 + (size_t)p.rows * 8 + 2 * kWaves * 8 + cap * 2 + n4 * 2 + n4 * 4 +

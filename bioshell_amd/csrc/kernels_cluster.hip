@@ -9,7 +9,7 @@
 // whose IEEE patterns order like unsigned integers).
 //
 // The agglomeration, two kernels per merge, for element counts beyond those of
-// the one-launch form (kernels_agglom.hip, up to about 16,000), follows
+// the one-launch form (kernels_agglom.hip, up to 16,384 elements), follows
 // bioshell-clustering/src/hierarchical/clustering_matrix.rs step for step on a
 // dense f32 matrix in HBM (see the comments at each phase); the merge sequence
 // it records is what the host rebuilds the tree from.

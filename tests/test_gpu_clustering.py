@@ -309,3 +309,92 @@ def test_launch_that_gives_up_leaves_the_call_to_the_stepwise_loop(gpu_ctx, monk
     want = O.hclust(up, n, linkage)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
+
+
+def device_merges_of(ctx, d_up, n, linkage):
+    """device_merges on a triangle in device memory."""
+    mi, mj, md = np.zeros(n - 1, np.uint32), np.zeros(n - 1, np.uint32), np.zeros(n - 1, np.float32)
+    B.check(_native.lib().bs_hierarchical_clustering_device(
+        ctx.handle, ctypes.c_void_p(d_up.data_ptr()), n, C.LINKAGES.index(linkage), mi.ctypes.data_as(_native.c_u32p),
+        mj.ctypes.data_as(_native.c_u32p), md.ctypes.data_as(_native.c_fp)))
+    return mi, mj, md
+
+
+@pytest.mark.parametrize("n,linkage,ties", [(11300, "average", False), (11300, "wards", True),
+                                            (13700, "complete", True), (13700, "centroid", False),
+                                            (15800, "average", True), (15800, "median", False),
+                                            (16384, "wards", False), (16384, "single", True)])
+def test_wide_blocks_equal_the_stepwise_loop(gpu_ctx, monkeypatch, n, linkage, ties):
+    """The element counts whose cached minima cover 128, 256 and 512 columns, up
+    to the largest of the one-launch loop: every merge and height of the
+    stepwise kernels (which the oracle covers at smaller counts), on random
+    values with few distinct ones or many, some of them never taken."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    k = n * (n - 1) // 2
+    up = torch.randint(1, 200, (k,), generator=g, device="cuda").float() if ties \
+        else torch.rand(k, generator=g, device="cuda") * 9 + 0.1
+    up[torch.randint(0, k, (k // 50,), generator=g, device="cuda")] = float("inf")
+    up[torch.randint(0, k, (k // 1000,), generator=g, device="cuda")] = float("nan")
+    torch.cuda.synchronize()
+    got = device_merges_of(gpu_ctx, up, n, linkage)
+    monkeypatch.setenv("BIOSHELL_CLUSTER_MAX_WAIT_MS", "0")
+    want = device_merges_of(gpu_ctx, up, n, linkage)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
+def test_stepwise_loop_above_the_one_launch_sizes(gpu_ctx):
+    """16,500 elements: the heights of points on a line by single linkage."""
+    n = 16500
+    rng = np.random.default_rng(n)
+    x = np.cumsum(rng.integers(1, 1000, n)).astype(np.float32)  # exact in f32, below 2^24
+    assert x[-1] < 2 ** 24
+    y = x[rng.permutation(n)]
+    up = np.concatenate([np.abs(y[i] - y[i + 1:]) for i in range(n - 1)])
+    mi, mj, md = device_merges(gpu_ctx, up, n, "single")
+    assert np.array_equal(md, np.sort(np.diff(x)))
+    assert (mi < mj).all() and (mj < n - np.arange(n - 1)).all()
+
+
+@pytest.mark.parametrize("n", [6200, 10000, 15800])
+def test_other_contexts_go_on_beside_a_clustering(gpu_ctx, n):
+    """One clustering leaves CUs to the rest of the device: the calls of another
+    context come back while it runs, none of them waiting for its end."""
+    import threading
+
+    import torch
+
+    L = 20
+    d_x = torch.from_numpy(B.generate_ensemble(n, n, L, sigma=(0.5, 3.0))).cuda()
+    up = torch.empty(n * (n - 1) // 2, dtype=torch.float32, device="cuda")
+    small = torch.empty(400 * 399 // 2, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    B.crmsd_all_vs_all_device(d_x.data_ptr(), n, L, up.data_ptr(), ctx=gpu_ctx)
+    gpu_ctx.synchronize()
+    device_merges_of(gpu_ctx, up, n, "average")
+    span, calls = [0.0, 0.0], []
+
+    def cluster():
+        span[0] = time.perf_counter()
+        device_merges_of(gpu_ctx, up, n, "average")
+        span[1] = time.perf_counter()
+
+    with B.Context(0) as other:
+        def call():
+            t0 = time.perf_counter()
+            B.crmsd_all_vs_all_device(d_x.data_ptr(), 400, L, small.data_ptr(), ctx=other)
+            other.synchronize()
+            calls.append(time.perf_counter() - t0)
+
+        call()
+        calls.clear()
+        th = threading.Thread(target=cluster)
+        th.start()
+        while th.is_alive():
+            call()
+        th.join()
+    took = span[1] - span[0]
+    print(f"clustering of {n}: {took * 1e3:.1f} ms, {len(calls)} calls beside it, the longest {max(calls) * 1e3:.2f} ms")
+    assert max(calls) < took / 4
