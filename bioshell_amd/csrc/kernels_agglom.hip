@@ -12,16 +12,18 @@
 //    column.
 //  - Every row caches its smallest entry per block of 64 columns (in LDS) and
 //    over the row.  A merge of slots I and J changes a row's entries at I, J
-//    and, by its new label, at L: a block is scanned again only if its cached
-//    minimum was at I or J, and the row's minimum is taken from the blocks only
-//    if it was.  With average linkage about one block scan per row and merge
-//    replaces a scan of the whole row, where the stepwise kernels read 67 MB a
-//    merge at 10,000 elements.
-//  - A row is read and written by one wave only, through ordinary cached
-//    accesses.  What a merge needs from other work-groups goes through small
-//    exchange buffers with agent-scope accesses: every work-group's best
-//    candidate (slots) and the merged row's new entries (newrow), each element's
-//    from the owner of its row.  Storing a candidate is also the arrival at
+//    and, by its new label, at L: the blocks of I and J are scanned again if
+//    their cached minimum was there, and the row's minimum is taken from the
+//    blocks only if it was.  With average linkage about one block scan per row
+//    and merge replaces a scan of the whole row, where the stepwise kernels read
+//    67 MB a merge at 10,000 elements.
+//  - A row belongs to one wave, which alone reads and writes it, through
+//    ordinary cached accesses; only the merged row is written by its whole
+//    work-group, a step's barrier before its wave reads it again.  What a merge
+//    needs from other work-groups goes through small exchange buffers with
+//    agent-scope accesses: every work-group's best candidate (slots) and the
+//    merged row's new entries (newrow), each element's from the owner of its
+//    row.  Storing a candidate is also the arrival at
 //    the step's barrier: everyone polls the slots until none is empty.  The
 //    buffers rotate by three: a work-group that has seen every candidate of
 //    step s knows that all have read those of step s - 1.
@@ -34,7 +36,7 @@
 // 1.3 us are the exchange and the rest the dependent steps of one wave, of 7.1
 // us at 10,000 (224 work-groups) about 3.4; memory traffic is below 0.5 TB/s.
 // Against two launches per merge: 300 elements 3.2 -> 1.3 ms, 2000 20 -> 10.5
-// ms, 10,000 190 -> 72 ms, 16,300 560 -> 240 ms (average linkage).  Measured and not kept: one
+// ms, 10,000 193 -> 71 ms, 16,300 745 -> 240 ms (average linkage).  Measured and not kept: one
 // work-group without the exchange (as fast up to 180 elements, slower above),
 // the matrix in LDS (3 % at 300 to 2000 elements), 8 waves per work-group (a
 // step is bound by the instructions of its waves).
@@ -54,7 +56,7 @@ constexpr int kMaxElements = 16384;     // labels take 14 bits of a published ke
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kWaves = 4;               // per work-group
 constexpr int kRowsWanted = 24;         // rows per work-group while the device has CUs for it
-constexpr int kWaveItems = 3 * 64;      // blocks a wave may have to scan again in a step
+constexpr int kWaveItems = 2 * 64;      // blocks a wave may have to scan again in a step
 constexpr int kUnroll = 4;              // block scans in flight per quarter wave
 constexpr int kCopy = 8;                // runs of a merged row in flight per quarter wave
 constexpr float kFltMax = 3.402823466e+38f;
@@ -296,14 +298,14 @@ __global__ __launch_bounds__(64 * kWaves) void agglom_kernel(AgglomArgs a)
             return (lq == i) | (lq == j);
         };
         const bool useJ = bJ != bI, useL = moved & (bL != bI) & (bL != bJ);  // uniform
-        const bool sI = scan & stale(kbI), sJ = scan & useJ & stale(kbJ), sL = scan & useL & stale(kbL);
-        const uint64_t mI = __ballot(sI), mJ = __ballot(sJ), mL = __ballot(sL);
-        const int nI = __popcll(mI), nJ = __popcll(mJ), n_items = nI + nJ + __popcll(mL);
+        // (a block without slots I and J caches neither's label)
+        const bool sI = scan & stale(kbI), sJ = scan & useJ & stale(kbJ);
+        const uint64_t mI = __ballot(sI), mJ = __ballot(sJ);
+        const int nI = __popcll(mI), n_items = nI + __popcll(mJ);
         if (n_items > 0) {
             const uint64_t below = (1ull << lane) - 1ull;
             if (sI) items[__popcll(mI & below)] = ((unsigned)r << 16) | (unsigned)bI;
             if (sJ) items[nI + __popcll(mJ & below)] = ((unsigned)r << 16) | (unsigned)bJ;
-            if (sL) items[nI + nJ + __popcll(mL & below)] = ((unsigned)r << 16) | (unsigned)bL;
             wave_lds_sync();
             for (int base = 0; base < n_items; base += 4 * kUnroll) {
                 int at[kUnroll], c0[kUnroll];
@@ -529,7 +531,7 @@ __global__ __launch_bounds__(256) void agglom_init_kernel(const float* __restric
 // elements 98.3 -> 100.6, 15,200 165 -> 172; 15,800, whose blocks widen for it,
 // 174 -> 240).  Blocks are 64 columns (one
 // 16-byte load of 16 lanes), wider only where the cached minima would not fit
-// the LDS: 128 from 11,201 elements, 256 from 13,557, 512 from 15,617.
+// the LDS: 128 from 11,201 elements, 256 from 13,601, 512 from 15,697.
 bool agglom_plan(int n, int n_cu, AgglomPlan* out)
 {
     if (n < 2 || n > kMaxElements) return false;
