@@ -34,7 +34,9 @@ bool exact_small(int n, int L, int n_cu);
 void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
                        hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
 // cRMSD of one pair of at most kPairMaxAtoms atoms, FP64, one launch; a, b and
-// out on the device or in pinned host memory.
+// out on the device or in pinned host memory.  The limit is what a work-group
+// holds in registers: a call of 3072 atoms takes 28 us, of 3100, with its copies
+// of pageable memory and the all-vs-all kernels, 353.
 constexpr int kPairMaxAtoms = 3072;
 void launch_pair(const double* a, const double* b, int L, double* out, hipStream_t s, uint64_t* clk = nullptr);
 int plain_block(int n, bool fp64, bool alone, int n_cu);

@@ -167,7 +167,10 @@ void bs_library_destroy(bs_library* lib)
 size_t bs_library_size(const bs_library* lib) { return lib ? (size_t)lib->P.n : 0; }
 size_t bs_library_atoms(const bs_library* lib) { return lib ? (size_t)lib->P.L : 0; }
 
-// Pinned bytes of a context for the queries and results of a small call.
+// Pinned bytes of a context for the queries and results of a small call.  What
+// limits them is the pinned memory a context holds: the calls are faster than
+// with copies up to there (against 25,000 x 256, k 100: 204 KB of queries 90
+// and 108 us, 1008 KB with 131 KB of results 168 and 181).
 constexpr size_t kStageQueries = 1 << 20, kStageResults = 256 << 10;
 
 static void check_query(bs_context* ctx, bs_library* lib, const double* q, size_t n_q)
