@@ -278,7 +278,7 @@ void enqueue_plain(bs_context* ctx, const Plan& P, const std::vector<const doubl
         launch_plain_batch(reinterpret_cast<const PlainEns*>(meta + o_ens[g]),
                            reinterpret_cast<const int*>(meta + o_pre[g]), (int)grp[g].size(),
                            pre[g].back(), 1 << g, fp64, s, launches == 0 ? rec->clk + kClkStart : nullptr,
-                           g == g_last ? rec->clk + kClkEnd : nullptr, rec->done);
+                           g == g_last ? rec->clk + kClkEnds : nullptr);
         ++launches;
     }
     BS_HIP(hipGetLastError());

@@ -130,6 +130,7 @@ bs_run_stats RunRecord::read() const
     // stream's work, which is none of the context's
     BS_HIP(hipMemcpyAsync(t, clk, sizeof(t), hipMemcpyDeviceToHost, stream));
     BS_HIP(hipStreamSynchronize(stream));
+    for (int k = 0; k < kClkEndWords; ++k) t[kClkEnd] = std::max(t[kClkEnd], t[kClkEnds + k * kClkEndStride]);
     auto ms = [&](int a, int b) { return t[b] > t[a] ? (double)(t[b] - t[a]) / khz : 0.0; };
     st.total_ms = ms(kClkStart, kClkEnd);
     if (kind == kOneStage) st.main_ms = st.total_ms;
@@ -217,7 +218,7 @@ void run_gram_with(const PrepView& A, const PrepView& B, const GramRun& run, con
                         g.triangle, A.n, run.out_ld, run.d_out, g.out_f64, run.h_count, run.st_min,
                         run.st_max, run.clk_resolve ? run.clk : nullptr, run.ends_call && !stats, s);
     if (stats)
-        launch_row_stats_decode(run.st_min, run.st_max, A.n, s, run.clk ? run.clk + kClkEnd : nullptr, run.done);
+        launch_row_stats_decode(run.st_min, run.st_max, A.n, s, run.clk ? run.clk + kClkEnds : nullptr);
     BS_HIP(hipGetLastError());
 }
 
@@ -331,10 +332,9 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
             }
         }
         if (exact)
-            launch_exact_avsa(d_xyz, n, L, d_out, out_f64, ctx->n_cu, ctx->prep.cent.as<double>(), s, rec->clk,
-                              rec->done);
+            launch_exact_avsa(d_xyz, n, L, d_out, out_f64, ctx->n_cu, ctx->prep.cent.as<double>(), s, rec->clk);
         else
-            launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s, rec->clk, rec->done);
+            launch_plain_avsa(d_xyz, n, L, m == BS_FP64_PLAIN, d_out, out_f64, ctx->n_cu, s, rec->clk);
         BS_HIP(hipGetLastError());
         rec->kind = RunRecord::kOneStage;
         rec->base.main_launches = 1;
@@ -345,7 +345,6 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
         run.d_out = d_out;
         run.out_f64 = out_f64;
         run.clk = rec->clk;
-        run.done = rec->done;
         if (fused) {
             // a second bank of tile results allows 32 x 32 tiles; an HBM
             // budget without room for it keeps the launch at 64 x 64 ones
@@ -382,13 +381,12 @@ void avsa_device(bs_context* ctx, const double* d_xyz, int n, int L, bs_method m
 bs::RunRecord* bs_context::begin_record()
 {
     if (ring.empty()) {
-        const size_t words = (kRing + 1 + bs::kBatchClocks + 1) * bs::kClkWords;
+        const size_t words = (kRing + 1 + bs::kBatchClocks) * bs::kClkWords;
         auto* clk = static_cast<uint64_t*>(ws_clock.ensure(words * 8, "call clocks"));
         bs::launch_zero_u32(reinterpret_cast<uint32_t*>(clk), (int)(2 * words), stream);
         BS_HIP(hipGetLastError());
         ring.resize(kRing);
         for (auto& r : ring) {
-            r.done = reinterpret_cast<unsigned*>(clk + words - bs::kClkWords);
             r.stream = stream;
             r.khz = clock_khz;
         }

@@ -105,7 +105,6 @@ struct GramRun {
     // re-evaluation's times and the call's end are taken in this run
     uint64_t* clk = nullptr;
     bool clk_main = true, clk_resolve = true, ends_call = true;
-    unsigned* done = nullptr;     // zero device word (with row statistics)
     bool triangle = true;
     void* d_out = nullptr;
     bool out_f64 = false;
@@ -162,7 +161,6 @@ struct RunRecord {
     // end (streamed blocks); all of them
     enum Kind { kUntimed, kOneStage, kTotalOnly, kTwoStages, kAllStages };
     uint64_t* clk = nullptr;      // kClkWords device words
-    unsigned* done = nullptr;     // zero device word for the last launch's stamp
     hipStream_t stream = nullptr;
     int khz = 0;                  // the clock's rate
     Kind kind = kUntimed;
@@ -245,10 +243,10 @@ struct bs_context {
     bs::QueryWorkspace qws;    // synchronous query calls
     std::vector<bs::RunRecord> ring;  // the last calls' records
     size_t ring_next = 0, ring_used = 0;
-    // clocks: kClkWords per record, those of the batch graphs (which write to
-    // the clock of their replay, not of a record), the calls' zero word
+    // clocks: kClkWords per record, then those of the batch graphs (which write
+    // to the clock of their replay, not of a record)
     bs::DevBuf ws_clock;
-    bs::Budget uncapped{0};            // ws_clock's 8 KiB: a capped context times its calls too
+    bs::Budget uncapped{0};            // ws_clock's 149 KB: a capped context times its calls too
     uint64_t batch_replays = 0;        // batch graphs launched, as the device counts them
     uint64_t* batch_clocks() { return ws_clock.as<uint64_t>() + kRing * bs::kClkWords; }
     static constexpr size_t kRing = 64;

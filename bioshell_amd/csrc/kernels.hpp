@@ -18,10 +18,9 @@ namespace bs {
 // (fp64), chosen by plain_block from the pair slots the tiles cover and, for
 // a lone launch (alone), from how many rounds of 2 work-groups per CU they
 // take on n_cu CUs.
-// clk (a call's clock, stamp.hpp) gets the launch's start and end; done is its
-// zero word.
+// clk (a call's clock, stamp.hpp) gets the launch's start and end.
 void launch_plain_avsa(const double* xyz, int n, int L, bool fp64, void* out, bool out_f64,
-                       int n_cu, hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
+                       int n_cu, hipStream_t s, uint64_t* clk = nullptr);
 // Sets the LDS limits of the kernels whose launches choose their size, on the
 // current device; before the first launch there.
 void exact_init();
@@ -32,7 +31,7 @@ void agglom_init();
 size_t exact_scratch_bytes(int n, int L, int n_cu);
 bool exact_small(int n, int L, int n_cu);
 void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
-                       hipStream_t s, uint64_t* clk = nullptr, unsigned* done = nullptr);
+                       hipStream_t s, uint64_t* clk = nullptr);
 // cRMSD of one pair of at most kPairMaxAtoms atoms, FP64, one launch; a, b and
 // out on the device or in pinned host memory.  The limit is what a work-group
 // holds in registers: a call of 3072 atoms takes 28 us, of 3100, with its copies
@@ -50,7 +49,7 @@ struct PlainEns {
 // Every ensemble of ens[0 .. n_ens) with block r in one launch: prefix (n_ens + 1
 // entries, device) counts their tiles, tiles = prefix[n_ens].
 void launch_plain_batch(const PlainEns* ens, const int* prefix, int n_ens, int tiles, int r, bool fp64,
-                        hipStream_t s, uint64_t* t_start, uint64_t* t_end, unsigned* done);
+                        hipStream_t s, uint64_t* t_start, uint64_t* t_end);
 
 // ------------------------------------------------------------ Gram path
 enum GramMode : int { kGramBF16x3 = 0, kGramFP32 = 1 };
@@ -211,7 +210,7 @@ size_t topk_scratch_bytes(int n_q, int n_lib, int k);
 // k for a given n_lib.
 bool topk_supported(int n_lib, int k);
 void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, float* val, void* scratch,
-                 hipStream_t s, uint64_t* t_end = nullptr, unsigned* done = nullptr);
+                 hipStream_t s, uint64_t* t_end = nullptr);
 
 // ------------------------------------------------------------ batches
 // One ensemble of a batch, as the batched kernels see it (device memory).
@@ -296,8 +295,7 @@ inline size_t fused_stats_tiles(int n)
 // Combines the epilogue's tile results into keys (kmin / kmax, n each, n >= 2),
 // which the resolve kernel then updates; decode turns the keys into f32.
 void launch_row_stats_combine(const unsigned* part, int banks, int n, unsigned* kmin, unsigned* kmax, hipStream_t s);
-void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end,
-                             unsigned* done);
+void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end);
 // For each of m members, the largest distance to the other members.
 void launch_members_row_max(const float* up, int n, const unsigned* members, int m, float* out,
                             hipStream_t s);

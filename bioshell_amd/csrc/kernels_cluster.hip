@@ -167,14 +167,14 @@ __global__ __launch_bounds__(512) void row_stats_reduce_kernel(const unsigned* _
 
 // Keys of elements [0, n) to f32 values, in place.
 __global__ void row_stats_decode_kernel(unsigned* __restrict__ kmin, unsigned* __restrict__ kmax, int n,
-                                        uint64_t* t_end, unsigned* done)
+                                        uint64_t* t_end)
 {
     const int e = blockIdx.x * 256 + threadIdx.x;
     if (e < n) {
         kmin[e] = fkey_inverse(kmin[e]);
         kmax[e] = fkey_inverse(kmax[e]);
     }
-    stamp_end(t_end, done);
+    stamp_end(t_end);
 }
 
 // Member a of the list: the largest distance to the other members (gather).
@@ -529,9 +529,9 @@ void launch_row_stats_combine(const unsigned* part, int banks, int n, unsigned* 
     row_stats_reduce_kernel<<<T, 512, 0, s>>>(part, banks, n, T, 0, T, 0, 1, 0, kmin, kmax);
 }
 
-void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end, unsigned* done)
+void launch_row_stats_decode(unsigned* kmin, unsigned* kmax, int n, hipStream_t s, uint64_t* t_end)
 {
-    row_stats_decode_kernel<<<(n + 255) / 256, 256, 0, s>>>(kmin, kmax, n, t_end, done);
+    row_stats_decode_kernel<<<(n + 255) / 256, 256, 0, s>>>(kmin, kmax, n, t_end);
 }
 
 void launch_members_row_max(const float* up, int n, const unsigned* members, int m, float* out,

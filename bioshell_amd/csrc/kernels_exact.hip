@@ -68,8 +68,7 @@ constexpr int kExactThreads = 256;
 
 __global__ __launch_bounds__(kExactThreads, 2) void exact_small_kernel(const double* __restrict__ xyz, int n, int L,
                                                                     int nt, void* __restrict__ out, int out_f64,
-                                                                    uint64_t* t_start, uint64_t* t_end,
-                                                                    unsigned* done)
+                                                                    uint64_t* t_start, uint64_t* t_end)
 {
     // sized by the launch (exact_small_lds): with a static array the compiler
     // sees one wave per SIMD and copies the accumulators between its two register
@@ -184,7 +183,7 @@ __global__ __launch_bounds__(kExactThreads, 2) void exact_small_kernel(const dou
             m[q] = (sm[q * 256 + t] + sm[(9 + q) * 256 + t]) + (sm[(18 + q) * 256 + t] + sm[(27 + q) * 256 + t]);
         store_pair(out, out_f64, n, i, j, exact_rmsd(m, cen[t >> 4][3], cen[16 + (t & 15)][3], L));
     }
-    stamp_end(t_end, done);
+    stamp_end(t_end);
 }
 
 // ------------------------------------------------------------ the rest
@@ -237,7 +236,7 @@ __device__ inline int exact_pos(int row, int c) { return (row * 64 + (c ^ row)) 
 __global__ __launch_bounds__(kExactThreads, 3) void exact_tile_kernel(const double* __restrict__ xyz, int n, int L,
                                                                       int nt, const double* __restrict__ cg,
                                                                       void* __restrict__ out, int out_f64,
-                                                                      uint64_t* t_end, unsigned* done)
+                                                                      uint64_t* t_end)
 {
     __shared__ __align__(16) double buf[2][kExactChunk * 3 * 64];
     int bi, bj;
@@ -332,7 +331,7 @@ __global__ __launch_bounds__(kExactThreads, 3) void exact_tile_kernel(const doub
         for (int q = 0; q < 9; ++q) m[q] = r == 0 ? acc[q][0] : r == 1 ? acc[q][1] : r == 2 ? acc[q][2] : acc[q][3];
         store_pair(out, out_f64, n, i, j, exact_rmsd(m, cg[4 * (int64_t)i + 3], gj, L));
     }
-    stamp_end(t_end, done);
+    stamp_end(t_end, kStampUniform);
 }
 
 constexpr int kLdsBytes = 160 * 1024;
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(256) void pair_kernel(const double* a, const double
 
 void launch_pair(const double* a, const double* b, int L, double* out, hipStream_t s, uint64_t* clk)
 {
-    pair_kernel<<<1, 256, 0, s>>>(a, b, L, out, clk ? clk + kClkStart : nullptr, clk ? clk + kClkEnd : nullptr);
+    pair_kernel<<<1, 256, 0, s>>>(a, b, L, out, clk ? clk + kClkStart : nullptr, clk ? clk + kClkEnds : nullptr);
 }
 
 // One launch while the LDS holds the coordinates (up to 211 atoms) and every
@@ -449,21 +448,21 @@ void exact_init()
 size_t exact_scratch_bytes(int n, int L, int n_cu) { return exact_small(n, L, n_cu) ? 0 : (size_t)n * 32; }
 
 void launch_exact_avsa(const double* xyz, int n, int L, void* out, bool out_f64, int n_cu, double* scratch,
-                       hipStream_t s, uint64_t* clk, unsigned* done)
+                       hipStream_t s, uint64_t* clk)
 {
     if (n < 2) return;
-    uint64_t *t0 = clk ? clk + kClkStart : nullptr, *t1 = clk ? clk + kClkEnd : nullptr;
+    uint64_t *t0 = clk ? clk + kClkStart : nullptr, *t1 = clk ? clk + kClkEnds : nullptr;
     const int f = out_f64 ? 1 : 0;
     if (exact_small(n, L, n_cu)) {
         const int nt = (n + 15) / 16, grid = nt * (nt + 1) / 2;
         const int lds = (int)exact_small_lds(L);
-        exact_small_kernel<<<grid, kExactThreads, lds, s>>>(xyz, n, L, nt, out, f, t0, t1, done);
+        exact_small_kernel<<<grid, kExactThreads, lds, s>>>(xyz, n, L, nt, out, f, t0, t1);
         return;
     }
     const int nt = (n + 31) / 32;
     exact_centre_kernel<<<(n + 3) / 4, 256, 0, s>>>(xyz, n, L, scratch, t0);
     exact_tile_kernel<<<(unsigned)((int64_t)nt * (nt + 1) / 2), kExactThreads, 0, s>>>(xyz, n, L, nt, scratch, out, f,
-                                                                                        t1, done);
+                                                                                        t1);
 }
 
 }  // namespace bs

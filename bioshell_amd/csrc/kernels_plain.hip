@@ -181,13 +181,13 @@ __device__ __forceinline__ void plain_tile(const double* __restrict__ xyz, int n
 template <class T, int R>
 __global__ __launch_bounds__(kThreads) void plain_kernel(const double* __restrict__ xyz, int n, int L,
                                                          int nt, void* __restrict__ out, int out_f64,
-                                                         uint64_t* t_start, uint64_t* t_end, unsigned* done)
+                                                         uint64_t* t_start, uint64_t* t_end)
 {
     stamp_start(t_start);
     int bi, bj;
     tri_tile(blockIdx.x, nt, bi, bj);
     plain_tile<T, R>(xyz, n, L, bi, bj, out, out_f64);
-    stamp_end(t_end, done);
+    stamp_end(t_end, kStampUniform);
 }
 
 // Many ensembles in one launch: block b is tile b - prefix[e] of ensemble e,
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kThreads) void plain_kernel(const double* __restric
 template <class T, int R>
 __global__ __launch_bounds__(kThreads) void plain_batch_kernel(const PlainEns* __restrict__ ens,
                                                                const int* __restrict__ prefix, int n_ens,
-                                                               uint64_t* t_start, uint64_t* t_end, unsigned* done)
+                                                               uint64_t* t_start, uint64_t* t_end)
 {
     stamp_start(t_start);
     const int b = blockIdx.x;
@@ -211,23 +211,23 @@ __global__ __launch_bounds__(kThreads) void plain_batch_kernel(const PlainEns* _
     int bi, bj;
     tri_tile(b - prefix[lo], E.nt, bi, bj);
     plain_tile<T, R>(E.xyz, E.n, E.L, bi, bj, E.out, 0);
-    stamp_end(t_end, done);
+    stamp_end(t_end);
 }
 
 template <class T, int R>
-void launch(const double* xyz, int n, int L, void* out, bool out_f64, hipStream_t s, uint64_t* clk, unsigned* done)
+void launch(const double* xyz, int n, int L, void* out, bool out_f64, hipStream_t s, uint64_t* clk)
 {
     const int nt = plain_tiles_per_side(n, R);
     plain_kernel<T, R><<<nt * (nt + 1) / 2, kThreads, 0, s>>>(xyz, n, L, nt, out, out_f64 ? 1 : 0,
                                                             clk ? clk + kClkStart : nullptr,
-                                                            clk ? clk + kClkEnd : nullptr, done);
+                                                            clk ? clk + kClkEnds : nullptr);
 }
 
 template <class T, int R>
 void launch_batch(const PlainEns* ens, const int* prefix, int n_ens, int tiles, hipStream_t s, uint64_t* t_start,
-                  uint64_t* t_end, unsigned* done)
+                  uint64_t* t_end)
 {
-    plain_batch_kernel<T, R><<<tiles, kThreads, 0, s>>>(ens, prefix, n_ens, t_start, t_end, done);
+    plain_batch_kernel<T, R><<<tiles, kThreads, 0, s>>>(ens, prefix, n_ens, t_start, t_end);
 }
 
 }  // namespace
@@ -256,41 +256,41 @@ int plain_block(int n, bool fp64, bool alone, int n_cu)
 }
 
 void launch_plain_avsa(const double* xyz, int n, int L, bool fp64, void* out, bool out_f64,
-                       int n_cu, hipStream_t s, uint64_t* clk, unsigned* done)
+                       int n_cu, hipStream_t s, uint64_t* clk)
 {
     if (n < 2) return;
     const int r = plain_block(n, fp64, true, n_cu);
     if (fp64) {
         if (r == 2)
-            launch<double, 2>(xyz, n, L, out, out_f64, s, clk, done);
+            launch<double, 2>(xyz, n, L, out, out_f64, s, clk);
         else
-            launch<double, 1>(xyz, n, L, out, out_f64, s, clk, done);
+            launch<double, 1>(xyz, n, L, out, out_f64, s, clk);
     } else {
         if (r == 4)
-            launch<float, 4>(xyz, n, L, out, out_f64, s, clk, done);
+            launch<float, 4>(xyz, n, L, out, out_f64, s, clk);
         else if (r == 2)
-            launch<float, 2>(xyz, n, L, out, out_f64, s, clk, done);
+            launch<float, 2>(xyz, n, L, out, out_f64, s, clk);
         else
-            launch<float, 1>(xyz, n, L, out, out_f64, s, clk, done);
+            launch<float, 1>(xyz, n, L, out, out_f64, s, clk);
     }
 }
 
 void launch_plain_batch(const PlainEns* ens, const int* prefix, int n_ens, int tiles, int r, bool fp64,
-                        hipStream_t s, uint64_t* t_start, uint64_t* t_end, unsigned* done)
+                        hipStream_t s, uint64_t* t_start, uint64_t* t_end)
 {
     if (n_ens == 0 || tiles == 0) return;
     if (fp64) {
         if (r == 2)
-            launch_batch<double, 2>(ens, prefix, n_ens, tiles, s, t_start, t_end, done);
+            launch_batch<double, 2>(ens, prefix, n_ens, tiles, s, t_start, t_end);
         else
-            launch_batch<double, 1>(ens, prefix, n_ens, tiles, s, t_start, t_end, done);
+            launch_batch<double, 1>(ens, prefix, n_ens, tiles, s, t_start, t_end);
     } else {
         if (r == 4)
-            launch_batch<float, 4>(ens, prefix, n_ens, tiles, s, t_start, t_end, done);
+            launch_batch<float, 4>(ens, prefix, n_ens, tiles, s, t_start, t_end);
         else if (r == 2)
-            launch_batch<float, 2>(ens, prefix, n_ens, tiles, s, t_start, t_end, done);
+            launch_batch<float, 2>(ens, prefix, n_ens, tiles, s, t_start, t_end);
         else
-            launch_batch<float, 1>(ens, prefix, n_ens, tiles, s, t_start, t_end, done);
+            launch_batch<float, 1>(ens, prefix, n_ens, tiles, s, t_start, t_end);
     }
 }
 

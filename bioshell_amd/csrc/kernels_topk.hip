@@ -193,8 +193,7 @@ __device__ inline void bitonic_sort(unsigned long long* s, int P)
 
 __global__ __launch_bounds__(1024) void topk_merge_kernel(const unsigned long long* __restrict__ cand, int m,
                                                           int k, uint32_t* __restrict__ out_idx,
-                                                          float* __restrict__ out_val, uint64_t* t_end,
-                                                          unsigned* done)
+                                                          float* __restrict__ out_val, uint64_t* t_end)
 {
     __shared__ unsigned long long s[kMergeMax];
     const int q = blockIdx.x, tid = threadIdx.x;
@@ -209,7 +208,7 @@ __global__ __launch_bounds__(1024) void topk_merge_kernel(const unsigned long lo
         out_idx[(int64_t)q * k + v] = (uint32_t)(c & 0xFFFFFFFFu);
         out_val[(int64_t)q * k + v] = __uint_as_float((uint32_t)(c >> 32));
     }
-    stamp_end(t_end, done);
+    stamp_end(t_end);
 }
 
 // One row in the registers of one work-group, KPT keys per thread (element
@@ -233,8 +232,7 @@ constexpr int kRowCand = 2048;
 template <int KPT>
 __global__ __launch_bounds__(kRowThreads) void topk_row_kernel(const float* __restrict__ scores, int n, int k,
                                                                uint32_t* __restrict__ out_idx,
-                                                               float* __restrict__ out_val, uint64_t* t_end,
-                                                               unsigned* done)
+                                                               float* __restrict__ out_val, uint64_t* t_end)
 {
     __shared__ __align__(16) unsigned long long cand[kRowCand];
     __shared__ uint32_t rank[kRowThreads];
@@ -401,7 +399,7 @@ __global__ __launch_bounds__(kRowThreads) void topk_row_kernel(const float* __re
         oi[v] = (uint32_t)(cand[v] & 0xFFFFFFFFu);
         ov[v] = __uint_as_float((uint32_t)(cand[v] >> 32));
     }
-    stamp_end(t_end, done);
+    stamp_end(t_end);
 }
 
 // Chunk length: at least kMinChunk, a multiple of 256, and few enough chunks
@@ -433,7 +431,7 @@ bool topk_supported(int n_lib, int k)
 }
 
 void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, float* val, void* scratch,
-                 hipStream_t s, uint64_t* t_end, unsigned* done)
+                 hipStream_t s, uint64_t* t_end)
 {
     if (n_q <= 0) return;
     if (k <= 0 || k > kTopkMax || k > n_lib) fail(BS_ERR_INVALID_ARGUMENT, "top-k: k = %d outside [1, min(%d, %d)]",
@@ -442,18 +440,18 @@ void launch_topk(const float* scores, int n_q, int n_lib, int k, uint32_t* idx, 
         fail(BS_ERR_UNSUPPORTED, "top-k: %d library members with k = %d exceed the selection's range", n_lib, k);
     if (n_lib <= kRowMax) {
         if (n_lib <= 8 * kRowThreads)
-            topk_row_kernel<8><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end, done);
+            topk_row_kernel<8><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end);
         else if (n_lib <= 16 * kRowThreads)
-            topk_row_kernel<16><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end, done);
+            topk_row_kernel<16><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end);
         else
-            topk_row_kernel<kRowKeys><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end, done);
+            topk_row_kernel<kRowKeys><<<n_q, kRowThreads, 0, s>>>(scores, n_lib, k, idx, val, t_end);
         return;
     }
     const int chunk = topk_chunk_len(n_lib, k);
     const int n_chunks = (n_lib + chunk - 1) / chunk;
     auto* cand = static_cast<unsigned long long*>(scratch);
     topk_chunk_kernel<<<dim3(n_chunks, n_q), kChunkThreads, 0, s>>>(scores, n_lib, k, chunk, cand);
-    topk_merge_kernel<<<n_q, 1024, 0, s>>>(cand, n_chunks * k, k, idx, val, t_end, done);
+    topk_merge_kernel<<<n_q, 1024, 0, s>>>(cand, n_chunks * k, k, idx, val, t_end);
 }
 
 }  // namespace bs

@@ -97,7 +97,7 @@ void enqueue_query(bs_library* lib, QueryWorkspace& ws, const double* q_host, in
         uint32_t* idx = stage.results ? stage.results : own;
         float* val = reinterpret_cast<float*>(idx + (size_t)n_q * k);
         launch_topk(scores, n_q, n_lib, k, idx, val, own + (size_t)n_q * k * 2, s,
-                    rec ? rec->clk + kClkEnd : nullptr, rec ? rec->done : nullptr);
+                    rec ? rec->clk + kClkEnds : nullptr);
         BS_HIP(hipGetLastError());
     }
     if (rec) {

@@ -563,3 +563,50 @@ def test_two_contexts_with_launches_of_different_lds_sizes():
         for t in th:
             t.join()
     assert not errors and got == [True, True]
+
+
+@pytest.mark.parametrize("method,n,L", [(B.Method.FP32_PLAIN, 600, 50), (B.Method.FP32_PLAIN, 1000, 20),
+                                        (B.Method.FP64_PLAIN, 200, 76)])
+def test_taking_times_does_not_slow_a_call(gpu_ctx, method, n, L):
+    """A launch of some hundred short work-groups, with its times taken and
+    without (the entry point that allocates nothing takes none): medians of 100
+    calls, to within a seventh."""
+    import ctypes
+    import time
+
+    import torch
+
+    d_x = torch.from_numpy(B.generate_ensemble(n, n, L, sigma=(0.5, 3.0))).cuda()
+    out = torch.zeros(n * (n - 1) // 2, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    f = B._native.lib().bs_crmsd_all_vs_all_device_noalloc, B._native.lib().bs_crmsd_all_vs_all_device
+
+    def call(which):
+        t0 = time.perf_counter()
+        B.check(f[which](gpu_ctx.handle, ctypes.c_void_p(d_x.data_ptr()), n, L, int(method),
+                         ctypes.c_void_p(out.data_ptr()), 0))
+        gpu_ctx.synchronize()
+        return time.perf_counter() - t0
+
+    t = np.median([[call(0), call(1)] for _ in range(120)][20:], axis=0)
+    print(f"{method.name} {n} x {L}: {t[0] * 1e6:.1f} us without times, {t[1] * 1e6:.1f} with them")
+    assert t[1] < t[0] * 8 / 7
+
+
+@pytest.mark.parametrize("method", [B.Method.FP64_PLAIN, B.Method.FP32_PLAIN])
+def test_times_of_launches_of_all_sizes(gpu_ctx, method):
+    """One work-group to more than take part in a launch's end: each call's
+    device time is its own, never the longer one's before it."""
+    import time
+
+    for n in (2, 17, 2500, 40, 5000, 2, 300):
+        x = B.generate_ensemble(n, n, 12, sigma=(0.5, 3.0))
+        B.crmsd_all_vs_all(x, method, ctx=gpu_ctx)
+        for _ in range(3):
+            t0 = time.perf_counter()
+            B.crmsd_all_vs_all(x, method, ctx=gpu_ctx)
+            wall = 1e3 * (time.perf_counter() - t0)
+            st = gpu_ctx.last_stats()
+            assert 0 < st["total_ms"] < wall and st["main_ms"] == st["total_ms"], (n, st, wall)
+    total = [h["total_ms"] for h in gpu_ctx.history(28)]
+    assert max(total[-8:]) < min(total[-12:-8])  # 5000 conformations, then 2 and 300
