@@ -41,8 +41,10 @@ uint64_t max_wait_ms()
 }
 
 // The one-launch loop.  False when the device would not take the launch (its
-// work-groups have to be resident together) or a work-group waited too long:
-// the caller runs the stepwise loop from the triangle, which is untouched.
+// work-groups have to be resident together), a work-group waited too long or the
+// budget has no room for its exchange buffers, which take 8 bytes an element
+// more than the stepwise loop's state: the caller runs the stepwise loop from
+// the triangle, which is untouched.
 bool cluster_one_launch(bs_context* ctx, const AgglomPlan& plan, const float* d_upper, size_t n, int rule,
                         uint32_t* merge_i, uint32_t* merge_j, float* merge_d)
 {
@@ -53,14 +55,20 @@ bool cluster_one_launch(bs_context* ctx, const AgglomPlan& plan, const float* d_
     aux.bind(&ctx->budget);
     const size_t ld = (n + 63) / 64 * 64;
     AgglomArgs a{};
-    a.D = static_cast<float*>(D.ensure(n * ld * 4, "clustering matrix"));
     a.ld = (int64_t)ld;
     a.n = N;
     a.rule = rule;
     // slots, status (with padding), merges, exchanged rows
     const size_t o_status = (size_t)plan.groups * 3 * 8, o_merge = o_status + 16,
                  o_new = (o_merge + n * 12 + 255) / 256 * 256;
-    char* p = static_cast<char*>(aux.ensure(o_new + ld * 12, "clustering state"));
+    char* p = nullptr;
+    try {
+        a.D = static_cast<float*>(D.ensure(n * ld * 4, "clustering matrix"));
+        p = static_cast<char*>(aux.ensure(o_new + ld * 12, "clustering state"));
+    } catch (const Error& e) {
+        if (e.code != BS_ERR_OUT_OF_BUDGET) throw;
+        return false;
+    }
     a.slots = reinterpret_cast<uint64_t*>(p);
     a.status = reinterpret_cast<unsigned*>(p + o_status);
     a.mi = reinterpret_cast<unsigned*>(p + o_merge);

@@ -398,3 +398,25 @@ def test_other_contexts_go_on_beside_a_clustering(gpu_ctx, n):
     took = span[1] - span[0]
     print(f"clustering of {n}: {took * 1e3:.1f} ms, {len(calls)} calls beside it, the longest {max(calls) * 1e3:.2f} ms")
     assert max(calls) < took / 4
+
+
+def test_budget_for_the_stepwise_loop_alone(gpu_ctx):
+    """A budget that holds the matrix and the stepwise kernels' state (16 bytes
+    an element and the candidates), but not the one-launch loop's exchange
+    buffers (24): the call runs.  Without room for the matrix it is refused."""
+    import torch
+
+    n, ld = 4000, 4032
+    g = torch.Generator(device="cuda").manual_seed(4)
+    up = torch.rand(n * (n - 1) // 2, generator=g, device="cuda") + 0.1
+    torch.cuda.synchronize()
+    want = device_merges_of(gpu_ctx, up, n, "average")
+    matrix = n * ld * 4 * 9 // 8  # buffers are an eighth larger than asked for
+    with B.Context(0, hbm_budget_bytes=matrix + 22 * n * 9 // 8) as ctx:
+        got = device_merges_of(ctx, up, n, "average")
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+    with B.Context(0, hbm_budget_bytes=matrix - 4096) as ctx:
+        with pytest.raises(B.BioshellGpuError) as e:
+            device_merges_of(ctx, up, n, "average")
+        assert e.value.status == -4
