@@ -183,10 +183,11 @@ __global__ __launch_bounds__(kThreads) void plain_kernel(const double* __restric
                                                          int nt, void* __restrict__ out, int out_f64,
                                                          uint64_t* t_start, uint64_t* t_end)
 {
-    stamp_start(t_start);
+    const uint64_t now = stamp_read();
     int bi, bj;
     tri_tile(blockIdx.x, nt, bi, bj);
     plain_tile<T, R>(xyz, n, L, bi, bj, out, out_f64);
+    stamp_store(t_start, now);
     stamp_end(t_end, kStampUniform);
 }
 
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void plain_batch_kernel(const PlainEns* _
                                                                const int* __restrict__ prefix, int n_ens,
                                                                uint64_t* t_start, uint64_t* t_end)
 {
-    stamp_start(t_start);
+    const uint64_t now = stamp_read();
     const int b = blockIdx.x;
     int lo = 0, hi = n_ens;
     while (hi - lo > 1) {
@@ -211,6 +212,7 @@ __global__ __launch_bounds__(kThreads) void plain_batch_kernel(const PlainEns* _
     int bi, bj;
     tri_tile(b - prefix[lo], E.nt, bi, bj);
     plain_tile<T, R>(E.xyz, E.n, E.L, bi, bj, E.out, 0);
+    stamp_store(t_start, now);
     stamp_end(t_end);
 }
 
